@@ -80,15 +80,15 @@ struct ScoreTables {
     double term_err = 0;      // measured error of the FP32 terms (k_term_error)
 };
 
-struct Ctl {                  // device control block
-    unsigned long long queue;
-    unsigned long long xq[8];     // per-XCD queues (fetch_xcd), right after the queue
-    unsigned long long best64;
-    unsigned long long checksum;
-    unsigned best32;
-    unsigned cand_count;      // candidates appended; with cand_over, CandOut::cand_count[0..1]
+struct Ctl {                  // device control block; hot words on lines of their own (QLINE)
+    unsigned long long queue[QLINE];
+    unsigned long long xq[8][QLINE];    // per-XCD queues (fetch_xcd), right after the queue
+    alignas(8 * QLINE) unsigned best32; // score bound
+    alignas(8 * QLINE) unsigned cand_count;   // candidates appended; with cand_over, CandOut::cand_count[0..1]
     unsigned cand_over;       // sticky overflow flag (the count can wrap past 2^32)
     unsigned bad_snp;         // lowest SNP with a sample in both planes (k_singles), or ~0
+    alignas(8 * QLINE) unsigned long long best64;
+    unsigned long long checksum;
 };
 static_assert(offsetof(Ctl, cand_over) == offsetof(Ctl, cand_count) + sizeof(unsigned),
               "the overflow flag follows the candidate count");
@@ -684,7 +684,7 @@ void fill_tri_common(episdet_dataset *ds, TriArgs &a)
     a.N1 = ds->N[1];
     a.singles = ds->singles;
     a.pairs = ds->pairs;
-    a.queue = &ds->ctl->queue;
+    a.queue = ds->ctl->queue;
     a.checksum = &ds->ctl->checksum;
     a.co.best_key = &ds->ctl->best32;
     a.co.cand_count = &ds->ctl->cand_count;
@@ -708,7 +708,7 @@ void fill_pair_common(episdet_dataset *ds, PairArgs &a, int T)
     a.singles = ds->singles;
     a.ntiles = (ds->n + T - 1) / T;
     a.nunits = (unsigned long long)a.ntiles * (a.ntiles + 1) / 2;
-    a.queue = &ds->ctl->queue;
+    a.queue = ds->ctl->queue;
     a.checksum = &ds->ctl->checksum;
     a.co.best_key = &ds->ctl->best32;
     a.co.cand_count = &ds->ctl->cand_count;
@@ -737,7 +737,7 @@ void fill_pairs(episdet_dataset *ds, PairArgs &a, bool mfma, int tile)
 // arguments, so no host memory has to outlive the call.
 int init_ctl(episdet_dataset *ds, unsigned long long u0 = 0, unsigned seed_key = 0)
 {
-    hipLaunchKernelGGL(k_init_search, dim3(1), dim3(64), 0, ds->stream, &ds->ctl->queue, &ds->ctl->best32,
+    hipLaunchKernelGGL(k_init_search, dim3(1), dim3(64), 0, ds->stream, ds->ctl->queue, &ds->ctl->best32,
                        &ds->ctl->cand_count, &ds->ctl->best64, &ds->ctl->checksum, u0, seed_key);
     HIPCHK(hipGetLastError());
     return EPISDET_OK;
@@ -2330,7 +2330,7 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         r.out_s64 = ds->cand_s64;
         rj[k].count = &ds->ctl->cand_count;
         rj[k].cap = batch_cap(opts[batched[k]], r.order, ktile[batched[k]]);
-        qp[k] = &ds->ctl->queue;
+        qp[k] = ds->ctl->queue;
         bp[k] = &ds->ctl->best32;
         cp[k] = &ds->ctl->cand_count;
     }
@@ -2341,8 +2341,8 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
     unsigned long long **d_qp = nullptr;
     unsigned **d_bp = nullptr, **d_cp = nullptr;
     constexpr int NQ = MFMA_TILES + MFMA_PAIR_TILES;   // one work queue per batched kernel
-    constexpr int QW = 9;                              // each: the queue, then 8 per-XCD queues
-    const unsigned long long zeros[NQ * QW] = {};
+    constexpr int QW = 9 * QLINE;                      // each: the queue, then 8 per-XCD queues
+    const std::vector<unsigned long long> zeros(NQ * QW, 0ull);
     for (int tl = 0; tl < MFMA_TILES; tl++) {
         CHK(dl.put(&d_ta[tl], ta[tl].data(), ta[tl].size()));
         CHK(dl.put(&d_tstart[tl], tstart[tl].data(), tstart[tl].size()));
@@ -2351,7 +2351,7 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         CHK(dl.put(&d_pa[tl], pa[tl].data(), pa[tl].size()));
         CHK(dl.put(&d_pstart[tl], pstart[tl].data(), pstart[tl].size()));
     }
-    CHK(dl.put(&d_bq, zeros, NQ * QW));
+    CHK(dl.put(&d_bq, zeros.data(), zeros.size()));
     CHK(dl.put(&d_rj, rj.data(), rj.size()));
     CHK(dl.put(&d_qp, qp.data(), qp.size()));
     CHK(dl.put(&d_bp, bp.data(), bp.size()));
