@@ -27,6 +27,10 @@ struct ScoreCtx {
     // clear above the best score before a set's FP32 score may be skipped
     // (2 margins plus the bound's own FP32 error)
     float lb_pi, lb_max, lb_scale, lb_slack, lb_lnw, lb_off, lb_top;
+    // quick_bound's forms of lb_scale and lb_lnw: the first widened by its
+    // roundings (0: no quick bound), the second per unit of its bit sum
+    float fb_scale, fb_lnw;
+    float tb_k, tb_a;   // its second bound's k(pi) and slope, scaled as lb_scale is
 };
 
 // Single-SNP counts of both classes: {cases c0, cases c1, controls c0,
@@ -154,6 +158,35 @@ __device__ __forceinline__ float k2_f32(const uint32_t *cas, const uint32_t *ctl
     return total - s;
 }
 
+// k2_f32 for the few sets of a unit that a bound did not rule out: three
+// cells a turn and no branch around a term's two forms, so nine table reads
+// and logarithms are in flight together (k2_f32 waits for each, about 900
+// cycles a cell).  The same operations in the same order: the same FP32 score.
+template <int NC>
+__device__ __forceinline__ float k2_f32_flat(const uint32_t *cas, const uint32_t *ctl, float invN, float k0, float c2,
+                                             float total, const float *s_lnf)
+{
+#pragma clang fp contract(off)
+    static_assert(NC % 3 == 0, "whole turns");
+    auto term = [&](uint32_t m) {
+        const float small = fmaf(-c2, (float)m, s_lnf[m < (uint32_t)LNF_SMALL ? m : 0u]);
+        const float x = (float)(m + 1u);
+        const float l2 = __builtin_amdgcn_logf(x * invN);
+        const float large = fmaf(fmaf(x, LN2_F, -0.5f * LN2_F), l2, k0);
+        return m < (uint32_t)LNF_SMALL ? small : large;
+    };
+    float s = 0.f, c = 0.f;
+#pragma unroll 1
+    for (int i = 0; i < NC; i += 3) {
+        float f[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) f[k] = (term(ctl[i + k]) + term(cas[i + k])) - term(ctl[i + k] + cas[i + k] + 1);
+#pragma unroll
+        for (int k = 0; k < 3; k++) kahan_add(s, c, f[k]);
+    }
+    return total - s;
+}
+
 // MI in FP32 from non-negative terms.  With x a cell's count in one class
 // and y = q n_c the count expected without association (q = Nc/N for the
 // cases, Nt/N for the controls, n_c = cases + controls of the cell),
@@ -275,6 +308,14 @@ __device__ __forceinline__ float badness_f32(const ScoreCtx &sc, const uint32_t 
     return -mi_f32(cas, ctl, sc.ncells, sc.mi_q, sc.mi_scale);
 }
 
+template <int NC>
+__device__ __forceinline__ float badness_f32_flat(const ScoreCtx &sc, const uint32_t *cas, const uint32_t *ctl,
+                                                  const float *s_lnf)
+{
+    if (sc.score == SCORE_K2) return k2_f32_flat<NC>(cas, ctl, sc.invN, sc.k0, sc.c, sc.k2_total, s_lnf);
+    return -mi_f32(cas, ctl, NC, sc.mi_q, sc.mi_scale);
+}
+
 // ---------------------------------------------------------------- FP64 --
 // Fixed operation sequences, no contraction: identical to the oracle's.
 
@@ -346,10 +387,14 @@ __device__ __forceinline__ float key2f(unsigned k)
 // upper bound of the k-th best, see publish_topk; it only decreases, so a
 // stale read only skips less) plus the slack, or +inf while no bound can
 // exceed it (bounds never exceed lb_top).
+__device__ __forceinline__ float skip_threshold(const ScoreCtx &sc, unsigned best)
+{
+    const float t = key2f(best) + sc.lb_slack;
+    return t < sc.lb_top ? t : INFINITY;
+}
 __device__ __forceinline__ float skip_threshold(const ScoreCtx &sc, const unsigned *best_key)
 {
-    const float t = key2f(__atomic_load_n(best_key, __ATOMIC_RELAXED)) + sc.lb_slack;
-    return t < sc.lb_top ? t : INFINITY;
+    return skip_threshold(sc, __atomic_load_n(best_key, __ATOMIC_RELAXED));
 }
 
 __device__ __forceinline__ unsigned long long d2key(double d)

@@ -16,19 +16,23 @@
 //    ahead.  KW = 16 (tile 3): 512-sample chunks, three buffers of 9 KB per
 //    class.  KW = 32 (tile 4): 1024-sample chunks, two buffers of 17 KB, so
 //    half as many barriers and load rounds per sample;
-//  * after the last chunk the accumulators go to LDS in two halves (Z 0-15,
-//    then 16-31) and the 256 threads score four triplets per half.
+//  * after the last chunk the accumulators go to LDS in two halves of 16 Y and
+//    each wave scores one X against 8 Y x 32 Z per half (s3_score).
 // LDS: at most 68 KB for the stage / dump area plus the ln m! table, so two
 // workgroups fit a CU.
 #pragma once
 #include "kernels_mfma3.hpp"
+#include "kernels_score3.hpp"
 
 namespace episdet {
 
 constexpr int M4_TY = 32, M4_TZ = 32;
-constexpr int M4_YROW = 4, M4_ZROW = 4 + 2 * M4_TY;         // X rows 0-3, then Y, then Z
+// X rows 0-3, then Y (2 y + plane), then Z by plane (32 plane + z): column
+// block cb of a tile is then plane cb of all 32 Z, so a lane holds both planes
+// of its Z and no counts move between lanes before scoring
+constexpr int M4_YROW = 4, M4_ZROW = 4 + 2 * M4_TY;
 constexpr int M4_ROWS = M4_ZROW + 2 * M4_TZ;                // 132 rows of a class
-constexpr int M4_DUMP_WORDS = 2 * 2 * 4 * 16 * 64;          // class x wave x tile x reg x lane (64 KB)
+constexpr int M4_DUMP_WORDS = 2 * 4 * S3_CLASS_WORDS;       // class x scoring wave x its counts (64 KB)
 
 // Chunk geometry, by words per row per chunk (KW):
 //  * KW 16 (512 samples): 64-byte rows, 16 rows per load, three buffers;
@@ -71,7 +75,7 @@ __device__ __forceinline__ void m4_row_offsets(int W, int X0, int y0, int z0, in
         int row;
         if (r < M4_YROW) row = 2 * X0 + r;
         else if (r < M4_ZROW) row = 2 * y0 + (r - M4_YROW);
-        else if (r < M4_ROWS) row = 2 * z0 + (r - M4_ZROW);
+        else if (r < M4_ROWS) row = 2 * (z0 + (r - M4_ZROW) % M4_TZ) + (r - M4_ZROW) / M4_TZ;
         else row = 2 * X0;                    // padding rows are never read
         roff[k] = ((unsigned)row * (unsigned)W + (unsigned)(q * 4)) * 4u;
     }
@@ -95,47 +99,53 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma4(BatchTri bt)
     using G = M4Geo<KW>;
     __shared__ __attribute__((aligned(16))) uint32_t smem[G::SMEM_WORDS];
     __shared__ unsigned long long s_u;
-    __shared__ float s_red[8];
+    __shared__ S3Pairs s_pairs;                         // scoring modes only
+    __shared__ unsigned s_best;
     __shared__ float s_lnf[scores_sets(MODE) ? LNF_SMALL : 1];
     if constexpr (scores_sets(MODE)) load_lnf(s_lnf);
     const int tid = threadIdx.x;
-    const int cls = tid >> 7, t = tid & 127;
-    const int xs = t >> 6, lane = t & 63, h = lane >> 5, i = lane & 31;
+    const int w = uniform(tid >> 6);                     // wave: 2 class + xs
+    const int cls = w >> 1, xs = w & 1;
     uint32_t *bufs = smem + cls * G::NBUF * G::BUF_WORDS;
-    // LDS rows read by this lane: its X's plane, Y rows of the four row
-    // blocks, Z rows of the two column blocks
-    const int xr = 2 * xs + ((i >> 1) & 1);
-    int yr[4];
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++) yr[rb] = M4_YROW + 2 * (rb * 8 + (i >> 2)) + (i & 1);
-    const int zr0 = M4_ZROW + i, zr1 = M4_ZROW + 32 + i;
     // loads per chunk issued by this wave
     const int my_loads = (G::LOADS - xs + 1) / 2;
 
     int g = 0, j = 0;
+    unsigned long long jfirst = 0, jend = 0;
+    TriArgs p;
+    if (tid == 0) s_u = atomicAdd(bt.queue, 1ull);
     for (;;) {
-        if (tid == 0) s_u = atomicAdd(bt.queue, 1ull);
         __syncthreads();
-        const unsigned long long uu = s_u;
+        const unsigned long long uu = uniform(s_u);
         if (uu >= bt.total) break;
         // job of this unit; a workgroup's units only increase
-        int jn = j;
-        while (jn + 1 < bt.njobs && bt.job_start[jn + 1] <= uu) jn++;
-        if (jn != j) {
-            j = jn;
+        if (uu >= jend) {
+            while (j + 1 < bt.njobs && ld_const(bt.job_start, (size_t)(j + 1)) <= uu) j++;
             g = 0;
+            p = ld_const(bt.jobs, (size_t)j);
+            jfirst = ld_const(bt.job_start, (size_t)j);
+            jend = ld_const(bt.job_start, (size_t)(j + 1));
         }
-        const TriArgs &p = bt.jobs[j];
-        const unsigned long long u = uu - bt.job_start[j];
+        const unsigned long long u = uu - jfirst;
         const uint32_t *base = cls ? p.p1 : p.p0;
         const int W = cls ? p.W1 : p.W0;
         const int nch_mine = W / KW;
         const int nch = (p.W0 > p.W1 ? p.W0 : p.W1) / KW;
-        g = next_group(p.gstart, p.ngroups, u, g);
-        const int X0 = 2 * (int)(u - p.gstart[g]);
-        const int2 gt = p.groups[g];
+        unsigned long long gfirst;
+        g = uniform_group(p.gstart, p.ngroups, u, g, &gfirst);
+        const int X0 = 2 * (int)(u - gfirst);
+        const int2 gt = ld_const(p.groups, (size_t)g);
         const int y0 = gt.x * M4_TY, z0 = gt.y * M4_TZ;
         const i32x4_t rsrc = m2_rsrc(base, cls ? p.bytes1 : p.bytes0);
+        // LDS rows read by this lane: its X's plane, Y rows of the four row
+        // blocks, Z rows of the two column blocks (made per unit: they are not
+        // to hold registers through the scoring)
+        const int lane = opaque(tid & 63), h = lane >> 5, i = lane & 31;
+        const int xr = 2 * xs + ((i >> 1) & 1);
+        int yr[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; rb++) yr[rb] = M4_YROW + 2 * (rb * 8 + (i >> 2)) + (i & 1);
+        const int zr0 = M4_ZROW + i, zr1 = M4_ZROW + 32 + i;
         unsigned roff[G::LOADS_PER_WAVE];
         m4_row_offsets<KW>(W, X0, y0, z0, xs, lane, roff);
 
@@ -152,6 +162,9 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma4(BatchTri bt)
 #pragma unroll
         for (int k = 0; k + 1 < G::NBUF; k++)
             if (k < nch_mine) m4_issue_buf<KW>(rsrc, roff, k * KW, lds_addr(bufs + k * G::BUF_WORDS), xs);
+        if constexpr (scores_sets(MODE)) s3_fill(p, X0, y0, z0, opaque(tid), s_pairs);
+        unsigned long long next = 0;
+        unsigned best = 0;
         for (int c = 0; c < nch; c++) {
             // this wave's loads of chunk c are done once at most those of the
             // chunks after it that are already issued (NBUF - 2 at most) are
@@ -166,6 +179,11 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma4(BatchTri bt)
             if (c + G::NBUF - 1 < nch_mine)
                 m4_issue_buf<KW>(rsrc, roff, (c + G::NBUF - 1) * KW,
                                  lds_addr(bufs + ((c + G::NBUF - 1) % G::NBUF) * G::BUF_WORDS), xs);
+            // the next unit's number and the score bound arrive while the last chunk is contracted
+            if (c + 1 == nch && tid == 0) {
+                next = atomicAdd(bt.queue, 1ull);
+                if constexpr (scores_sets(MODE)) best = __hip_atomic_load(p.co.best_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             if (c < nch_mine) {
                 const uint32_t *cur = bufs + (c % G::NBUF) * G::BUF_WORDS;
                 // the words of slice s + 1 are read once the class-3
@@ -203,71 +221,55 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma4(BatchTri bt)
             }
         }
         __builtin_amdgcn_s_waitcnt(0);
+        if (tid == 0) {
+            s_u = next;
+            s_best = best;
+        }
         __syncthreads();
 
-        float bad[8];
-        unsigned long long packed[8];
+        // Scoring wave w takes X0 + w/2 and, of each half, row block w%2; half
+        // hf holds row blocks 2 hf and 2 hf + 1 of every wave
+        const int txs = w >> 1, rbl = w & 1;
+        const int ln = opaque(tid & 63), eh = ln >> 5, ei = ln & 31;
+        const int X = X0 + txs, Z = z0 + ei;
+        S3Yz yz{};
         unsigned long long hsum = 0;
         // Sets whose badness lower bound exceeds the best FP32 score found so
         // far by more than the slack cannot become candidates; their FP32
         // score is skipped (skip_threshold).
         float skip_above = INFINITY;
-        if constexpr (scores_sets(MODE)) skip_above = skip_threshold(p.sc, p.co.best_key);
+        if constexpr (scores_sets(MODE)) {
+            skip_above = skip_threshold(p.sc, s_best);
+            s3_yz(p, y0 + rbl * 8 + eh, Z, yz);
+        }
+        float *dump = (float *)smem;
+        // -> LDS [cls][xs][row block of the half][q][k][lane][ij]
+        auto put = [&](const v16f_t &v, int b, int cb) {
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-            // column block hf of every row block -> LDS [cls][xs][rb][reg][lane]
+            for (int q = 0; q < 4; q++)
+                *(float4 *)&dump[((cls * 2 + xs) * 2 + b) * S3_CLASS_WORDS + ((q * 2 + cb) * 64 + ln) * 4] =
+                    make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        };
 #pragma unroll
-            for (int rb = 0; rb < 4; rb++)
+        for (int b = 0; b < 2; b++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    smem[((((cls * 2 + xs) * 4 + rb) * 16) + r) * 64 + lane] = (uint32_t)acc[rb][hf][r];
+            for (int cb = 0; cb < 2; cb++) put(acc[b][cb], b, cb);
+        __syncthreads();
+        // rolled, so the kernel holds the scoring code once
+#pragma unroll 1
+        for (int hf = 0;; hf++) {
+            const int yl = (2 * hf + rbl) * 8;
+            s3_score<MODE>(p, dump + w * S3_CLASS_WORDS, 4 * S3_CLASS_WORDS, s_pairs, s_pairs.xy + (txs * 32 + yl) * 12,
+                           txs * 32 + ei, yz, X, y0 + yl, Z, ln, skip_above, s_lnf, hsum);
+            if (hf) break;
+            if constexpr (scores_sets(MODE)) s3_yz(p, y0 + (2 + rbl) * 8 + eh, Z, yz);
             __syncthreads();
 #pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                const int m = hf * 4 + q4;
-                const int T = q4 * 256 + tid;                   // 2 X x 32 Y x 16 Z of this half
-                const int txs = T >> 9, yl = (T >> 4) & 31, zl = hf * 16 + (T & 15);
-                const int X = X0 + txs, Y = y0 + yl, Z = z0 + zl;
-                bad[m] = INFINITY;
-                packed[m] = (unsigned long long)X | ((unsigned long long)Y << 21) | ((unsigned long long)Z << 42);
-                if (!(X < Y && Y < Z && Z < p.n)) continue;
-                // tile row 4*y8 + ij of row block yl/8 in wave (class, txs);
-                // tile column 2*(zl%16) + k.  Output register
-                // r = 4*(row/8) + row%4 of lane 32*((row/4)%2) + column.
-                const int trb = yl >> 3, y8 = yl & 7;
-                const int z16 = zl & 15;
-                uint32_t n8c[8], n8t[8];
+            for (int b = 0; b < 2; b++)
 #pragma unroll
-                for (int ij = 0; ij < 4; ij++)
-#pragma unroll
-                    for (int kk = 0; kk < 2; kk++) {
-                        const int reg = 4 * (y8 >> 1) + ij;
-                        const int ln = 32 * (y8 & 1) + 2 * z16 + kk;
-                        const int off = ((trb * 16) + reg) * 64 + ln;
-                        n8c[ij * 2 + kk] = smem[(0 * 2 + txs) * 4 * 16 * 64 + off];
-                        n8t[ij * 2 + kk] = smem[(1 * 2 + txs) * 4 * 16 * 64 + off];
-                    }
-                const Singles sx = ld_global(p.singles, X), sy = ld_global(p.singles, Y);
-                uint32_t cas[27], ctl[27];
-                triplet_tables(p, X, Y, Z, sx, sy, n8c, n8t, cas, ctl);
-                if constexpr (scores_sets(MODE)) {
-                    if (skip_above < INFINITY && bound_exceeds<27>(p.sc, cas, ctl, skip_above))
-                        continue;                           // bad[m] stays INFINITY
-                    bad[m] = badness_f32(p.sc, cas, ctl, s_lnf);
-                } else if constexpr (MODE == MODE_DUMP) {
-                    uint32_t *o = p.dump + rank3(X, Y, Z) * 54;
-                    for (int c = 0; c < 27; c++) {
-                        o[c] = cas[c];
-                        o[27 + c] = ctl[c];
-                    }
-                } else if constexpr (MODE == MODE_CHECKSUM) {
-                    hsum += table_hash(rank3(X, Y, Z), cas, ctl, 27);
-                }
-            }
+                for (int cb = 0; cb < 2; cb++) put(acc[2 + b][cb], b, cb);
             __syncthreads();
         }
-        if constexpr (MODE == MODE_SEARCH) publish_candidates<8, 4>(p.co, p.sc.margin, bad, packed, s_red);
-        if constexpr (MODE == MODE_TOPK) publish_topk<8, 4>(p.co, p.sc.margin, bad, packed);
         if constexpr (MODE == MODE_CHECKSUM) {
             if (hsum) atomicAdd(p.checksum, hsum);
         }

@@ -4,7 +4,7 @@
 // Version 4 runs its cases and controls waves side by side, two of each per
 // workgroup, so when one class holds more samples than the other, the waves
 // of the smaller class (and the SIMDs they run on) finish early.  This
-// version keeps version 4's unit and epilogue and gives every wave a share
+// version keeps version 4's unit and scoring and gives every wave a share
 // of both classes:
 //  * work unit: (X, X+1) x 32 Y x 32 Z;
 //  * 256 threads = 4 waves; wave w contracts X + w/2 against Y row blocks
@@ -15,8 +15,8 @@
 //    64 Y + 64 Z rows of 128 bytes, loaded straight to LDS through its
 //    class's scalar buffer descriptor into one of three buffers, two chunks
 //    ahead, each wave waiting only for its own loads;
-//  * after the last chunk the accumulators go to LDS in two halves (Z 0-15,
-//    then 16-31) and the 256 threads score four triplets per half.
+//  * after the last chunk each wave scores its own counts, through LDS in two
+//    halves of 8 Y (s3_score).
 // Each A operand feeds two MFMAs instead of version 4's four, so the operand
 // work per MFMA is higher; AUTO picks this version when the classes differ
 // in size (see choose_kernel).
@@ -34,7 +34,7 @@ constexpr int M5_LOADS_PER_WAVE = (M5_LOADS + 3) / 4;       // 5 (wave 0) or 4
 constexpr int M5_BUF_WORDS = M5_LOADS * M5_ROWS_PER_LOAD * M5_KW;              // 4352 (17 KB)
 constexpr int M5_NBUF = 3;
 constexpr int M5_STAGE_WORDS = M5_NBUF * M5_BUF_WORDS;
-constexpr int M5_DUMP_WORDS = 2 * 4 * 2 * 16 * 64;          // class x wave x row block x reg x lane (64 KB)
+constexpr int M5_DUMP_WORDS = 2 * 4 * S3_CLASS_WORDS;       // class x wave x its counts (64 KB)
 constexpr int M5_SMEM_WORDS = M5_STAGE_WORDS > M5_DUMP_WORDS ? M5_STAGE_WORDS : M5_DUMP_WORDS;
 static_assert(M5_KW == M2_KW, "128-byte rows use the swizzle of m2_at");
 
@@ -51,7 +51,7 @@ __device__ __forceinline__ void m5_row_offsets(int W, int X0, int y0, int z0, in
         int row;
         if (r < M4_YROW) row = 2 * X0 + r;
         else if (r < M4_ZROW) row = 2 * y0 + (r - M4_YROW);
-        else if (r < M4_ROWS) row = 2 * z0 + (r - M4_ZROW);
+        else if (r < M4_ROWS) row = 2 * (z0 + (r - M4_ZROW) % M4_TZ) + (r - M4_ZROW) / M4_TZ;
         else row = 2 * X0;                    // padding rows are never read
         roff[k] = ((unsigned)row * (unsigned)W + (unsigned)(q * 4)) * 4u;
     }
@@ -106,43 +106,49 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma5(BatchTri bt)
 {
     __shared__ __attribute__((aligned(16))) uint32_t smem[M5_SMEM_WORDS];
     __shared__ unsigned long long s_u;
-    __shared__ float s_red[8];
+    __shared__ S3Pairs s_pairs;                         // scoring modes only
+    __shared__ unsigned s_best;
     __shared__ float s_lnf[scores_sets(MODE) ? LNF_SMALL : 1];
     if constexpr (scores_sets(MODE)) load_lnf(s_lnf);
     const int tid = threadIdx.x;
-    const int w = tid >> 6, lane = tid & 63, h = lane >> 5, i = lane & 31;
+    const int w = uniform(tid >> 6);
     const int xs = w >> 1, yh = w & 1;
-    // LDS rows read by this lane: its X's plane, Y rows of its two row
-    // blocks, Z rows of the two column blocks
-    const int xr = 2 * xs + ((i >> 1) & 1);
-    int yr[2];
-#pragma unroll
-    for (int rl = 0; rl < 2; rl++) yr[rl] = M4_YROW + 2 * ((2 * yh + rl) * 8 + (i >> 2)) + (i & 1);
-    const int zr0 = M4_ZROW + i, zr1 = M4_ZROW + 32 + i;
     // loads per chunk issued by this wave
     const int my_loads = (M5_LOADS - w + 3) / 4;
 
     int g = 0, j = 0;
+    unsigned long long jfirst = 0, jend = 0;
+    TriArgs p;
+    if (tid == 0) s_u = atomicAdd(bt.queue, 1ull);
     for (;;) {
-        if (tid == 0) s_u = atomicAdd(bt.queue, 1ull);
         __syncthreads();
-        const unsigned long long uu = s_u;
+        const unsigned long long uu = uniform(s_u);
         if (uu >= bt.total) break;
         // job of this unit; a workgroup's units only increase
-        int jn = j;
-        while (jn + 1 < bt.njobs && bt.job_start[jn + 1] <= uu) jn++;
-        if (jn != j) {
-            j = jn;
+        if (uu >= jend) {
+            while (j + 1 < bt.njobs && ld_const(bt.job_start, (size_t)(j + 1)) <= uu) j++;
             g = 0;
+            p = ld_const(bt.jobs, (size_t)j);
+            jfirst = ld_const(bt.job_start, (size_t)j);
+            jend = ld_const(bt.job_start, (size_t)(j + 1));
         }
-        const TriArgs &p = bt.jobs[j];
-        const unsigned long long u = uu - bt.job_start[j];
+        const unsigned long long u = uu - jfirst;
         const int nch0 = p.W0 / M5_KW, nch = nch0 + p.W1 / M5_KW;
-        g = next_group(p.gstart, p.ngroups, u, g);
-        const int X0 = 2 * (int)(u - p.gstart[g]);
-        const int2 gt = p.groups[g];
+        unsigned long long gfirst;
+        g = uniform_group(p.gstart, p.ngroups, u, g, &gfirst);
+        const int X0 = 2 * (int)(u - gfirst);
+        const int2 gt = ld_const(p.groups, (size_t)g);
         const int y0 = gt.x * M4_TY, z0 = gt.y * M4_TZ;
         const i32x4_t rs0 = m2_rsrc(p.p0, p.bytes0), rs1 = m2_rsrc(p.p1, p.bytes1);
+        // LDS rows read by this lane: its X's plane, Y rows of its two row
+        // blocks, Z rows of the two column blocks (made per unit: they are not
+        // to hold registers through the scoring)
+        const int lane = opaque(tid & 63), h = lane >> 5, i = lane & 31;
+        const int xr = 2 * xs + ((i >> 1) & 1);
+        int yr[2];
+#pragma unroll
+        for (int rl = 0; rl < 2; rl++) yr[rl] = M4_YROW + 2 * ((2 * yh + rl) * 8 + (i >> 2)) + (i & 1);
+        const int zr0 = M4_ZROW + i, zr1 = M4_ZROW + 32 + i;
         unsigned roff0[M5_LOADS_PER_WAVE], roff1[M5_LOADS_PER_WAVE];
         m5_row_offsets(p.W0, X0, y0, z0, w, lane, roff0);
         m5_row_offsets(p.W1, X0, y0, z0, w, lane, roff1);
@@ -168,6 +174,9 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma5(BatchTri bt)
                 else m5_issue_buf(rs1, roff1, (k - nch0) * M5_KW, lds_addr(nb), w);
             }
         }
+        if constexpr (scores_sets(MODE)) s3_fill(p, X0, y0, z0, opaque(tid), s_pairs);
+        unsigned long long next = 0;
+        unsigned best = 0;
         // two loops, one per class, so each contracts into one fixed set of
         // accumulators
 #pragma unroll
@@ -188,79 +197,62 @@ __global__ __launch_bounds__(256, 2) void k_triplets_mfma5(BatchTri bt)
                     if (tn < nch0) m5_issue_buf(rs0, roff0, tn * M5_KW, lds_addr(nb), w);
                     else m5_issue_buf(rs1, roff1, (tn - nch0) * M5_KW, lds_addr(nb), w);
                 }
+                // the next unit's number and the score bound arrive while the last chunk is contracted
+                if (t + 1 == nch && tid == 0) {
+                next = atomicAdd(bt.queue, 1ull);
+                if constexpr (scores_sets(MODE)) best = __hip_atomic_load(p.co.best_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
                 m5_chunk(smem + (t % M5_NBUF) * M5_BUF_WORDS, xr, yr, zr0, zr1, h, acc[c], bt.sh);
             }
         }
         __builtin_amdgcn_s_waitcnt(0);
+        if (tid == 0) {
+            s_u = next;
+            s_best = best;
+        }
         __syncthreads();
 
-        float bad[8];
-        unsigned long long packed[8];
+        // Each wave scores what it counted: half hf holds its row block hf
+        const int ln = opaque(tid & 63), eh = ln >> 5, ei = ln & 31;
+        const int X = X0 + xs, Z = z0 + ei;
+        S3Yz yz{};
         unsigned long long hsum = 0;
         // Sets whose badness lower bound exceeds the best FP32 score found so
         // far by more than the slack cannot become candidates; their FP32
         // score is skipped (skip_threshold).
         float skip_above = INFINITY;
-        if constexpr (scores_sets(MODE)) skip_above = skip_threshold(p.sc, p.co.best_key);
+        if constexpr (scores_sets(MODE)) {
+            skip_above = skip_threshold(p.sc, s_best);
+            s3_yz(p, y0 + 2 * yh * 8 + eh, Z, yz);
+        }
+        float *dump = (float *)smem;
+        // -> LDS [class][wave][q][k][lane][ij], read by this wave alone
+        auto put = [&](const v16f_t &v, int c, int cb) {
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-            // column block hf -> LDS [class][wave][row block][reg][lane]
+            for (int q = 0; q < 4; q++)
+                *(float4 *)&dump[(c * 4 + w) * S3_CLASS_WORDS + ((q * 2 + cb) * 64 + ln) * 4] =
+                    make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        };
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++) put(acc[c][0][cb], c, cb);
+        __builtin_amdgcn_wave_barrier();
+        // rolled, so the kernel holds the scoring code once
+#pragma unroll 1
+        for (int hf = 0;; hf++) {
+            const int yl = (2 * yh + hf) * 8;
+            s3_score<MODE>(p, dump + w * S3_CLASS_WORDS, 4 * S3_CLASS_WORDS, s_pairs, s_pairs.xy + (xs * 32 + yl) * 12,
+                           xs * 32 + ei, yz, X, y0 + yl, Z, ln, skip_above, s_lnf, hsum);
+            if (hf) break;
+            if constexpr (scores_sets(MODE)) s3_yz(p, y0 + (2 * yh + 1) * 8 + eh, Z, yz);
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int c = 0; c < 2; c++)
 #pragma unroll
-                for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        smem[((((c * 4 + w) * 2 + rb) * 16) + r) * 64 + lane] = (uint32_t)acc[c][rb][hf][r];
-            __syncthreads();
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                const int m = hf * 4 + q4;
-                const int T = q4 * 256 + tid;                   // 2 X x 32 Y x 16 Z of this half
-                const int txs = T >> 9, yl = (T >> 4) & 31, zl = hf * 16 + (T & 15);
-                const int X = X0 + txs, Y = y0 + yl, Z = z0 + zl;
-                bad[m] = INFINITY;
-                packed[m] = (unsigned long long)X | ((unsigned long long)Y << 21) | ((unsigned long long)Z << 42);
-                if (!(X < Y && Y < Z && Z < p.n)) continue;
-                // row block yl/8 = 2*yh + rbl lives in wave 2*txs + yh as its
-                // row block rbl; tile row 4*y8 + ij, tile column 2*(zl%16) + k.
-                // Output register r = 4*(row/8) + row%4 of lane
-                // 32*((row/4)%2) + column.
-                const int rbg = yl >> 3, y8 = yl & 7;
-                const int tw = 2 * txs + (rbg >> 1), rbl = rbg & 1;
-                const int z16 = zl & 15;
-                uint32_t n8c[8], n8t[8];
-#pragma unroll
-                for (int ij = 0; ij < 4; ij++)
-#pragma unroll
-                    for (int kk = 0; kk < 2; kk++) {
-                        const int reg = 4 * (y8 >> 1) + ij;
-                        const int ln = 32 * (y8 & 1) + 2 * z16 + kk;
-                        const int off = (((tw * 2 + rbl) * 16) + reg) * 64 + ln;
-                        n8c[ij * 2 + kk] = smem[0 * 4 * 2 * 16 * 64 + off];
-                        n8t[ij * 2 + kk] = smem[1 * 4 * 2 * 16 * 64 + off];
-                    }
-                const Singles sx = ld_global(p.singles, X), sy = ld_global(p.singles, Y);
-                uint32_t cas[27], ctl[27];
-                triplet_tables(p, X, Y, Z, sx, sy, n8c, n8t, cas, ctl);
-                if constexpr (scores_sets(MODE)) {
-                    if (skip_above < INFINITY && bound_exceeds<27>(p.sc, cas, ctl, skip_above))
-                        continue;                           // bad[m] stays INFINITY
-                    bad[m] = badness_f32(p.sc, cas, ctl, s_lnf);
-                } else if constexpr (MODE == MODE_DUMP) {
-                    uint32_t *o = p.dump + rank3(X, Y, Z) * 54;
-                    for (int c = 0; c < 27; c++) {
-                        o[c] = cas[c];
-                        o[27 + c] = ctl[c];
-                    }
-                } else if constexpr (MODE == MODE_CHECKSUM) {
-                    hsum += table_hash(rank3(X, Y, Z), cas, ctl, 27);
-                }
-            }
-            __syncthreads();
+                for (int cb = 0; cb < 2; cb++) put(acc[c][1][cb], c, cb);
+            __builtin_amdgcn_wave_barrier();
         }
-        if constexpr (MODE == MODE_SEARCH) publish_candidates<8, 4>(p.co, p.sc.margin, bad, packed, s_red);
-        if constexpr (MODE == MODE_TOPK) publish_topk<8, 4>(p.co, p.sc.margin, bad, packed);
         if constexpr (MODE == MODE_CHECKSUM) {
             if (hsum) atomicAdd(p.checksum, hsum);
         }

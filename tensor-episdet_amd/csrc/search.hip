@@ -392,6 +392,30 @@ ScoreCtx make_ctx(const episdet_dataset *ds, int score, int order)
     sc.lb_lnw = (float)lnw;
     sc.lb_off = (float)off;
     sc.lb_top = (float)top;
+    // quick_bound (FP32 cells): with M = sqrt(S N), every marginal's |D| is at
+    // most M (Cauchy-Schwarz), so a base cell or marginal errs by at most u M
+    // and a cell derived from errors e1 + e2 + e3 by at most that plus 3 u M:
+    // over the 27 cells 1 (8 of them), 6 (12), 16 (6) and 36 (1) times u M,
+    // 57.3 u M in the 2-norm (9 cells: below that).  With T >= 1 below D^2 / T,
+    // sqrt(S') >= sqrt(S) (1 - 57.3 u sqrt(N)); the sum's own roundings are
+    // under 1e-5.  Cell totals and the sum of their bits are exact below 2^23
+    // samples; with more, the quick bound is off.
+    const double eta = 57.3 * u * std::sqrt((double)N);
+    const bool quick = N < (1 << 23) && (score != EPISDET_SCORE_K2 || lnw > 0.0);
+    sc.fb_scale = quick ? (float)(scale / ((1.0 - eta) * (1.0 - eta)) * (1.0 + 1e-5)) : 0.f;
+    sc.fb_lnw = (float)(lnw * std::ldexp(1.0, -23));
+    // Second bound, sum of f(D) = D^2 r (k + a r |D|) over the cells: f is
+    // convex in |D| with |D| f' <= 3 f, so with cells off by delta the sum
+    // loses at most 3 sum |delta| r |D| w <= 3 sqrt(1.125 wmax) |delta| sqrt(sum f)
+    // (Cauchy-Schwarz; r <= 1.125, w = k + a r |D| <= wmax = k + 1.125 a), and
+    // |delta| <= eta sqrt(S) <= eta sqrt(sum f / k).
+    const double kpi = 1.0 / (2.0 * qc * qt);
+    const double slope = std::max({0.0, (-std::log1p(-qc) / (qc * qc) - kpi) / qc, (-std::log(qc) / (qt * qt) - kpi) / qt});
+    const double loss = 3.0 * eta * std::sqrt(1.125 * (1.0 + 1.125 * slope / kpi));
+    const double widen = scale / K * (1.0 + 1e-6) / (1.0 - loss) * (1.0 + 1e-5);
+    // (a class of a few samples among many: the second bound rules out nothing)
+    sc.tb_k = loss < 0.5 ? (float)(kpi * widen) : 1e30f;
+    sc.tb_a = loss < 0.5 ? (float)(slope * widen) : 0.f;
     sc.lb_slack = (float)(2.0 * sc.margin + scale * ncells * 8.0 * ulp32((double)N) + extra);
     return sc;
 }
@@ -1062,6 +1086,12 @@ int issue_fused(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned long long
     if (order == 3 && mfma) CHK(upload_single(ds, ta, ta.nunits));
     else if (order == 2) CHK(upload_single(ds, pa, pa.nunits));
     CHK(init_ctl(ds, u0, seed_key));
+    // the 3-way kernels that tighten the top-k bound from the candidates' own
+    // scores (tighten_topk) must find +inf in slots not written yet
+    if (topk && order == 3 && mfma && tile >= 3) {
+        hipLaunchKernelGGL(k_fill_f32, dim3(4 * ds->cu), dim3(256), 0, ds->stream, ds->cand_s32, cap, INFINITY);
+        HIPCHK(hipGetLastError());
+    }
     HIPCHK(hipEventRecord(e0, ds->stream));
     if (topk)
         rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_TOPK>(ds, tile, ta, ds->stream, false)

@@ -1,0 +1,30 @@
+"""Scoring of the 3-way kernels' work units (MFMA tiles 3, 4 and 5): the sets
+at the edges of a unit (X pairs, 32 Y, 32 Z), classes of one and several
+chunks, and the top-k bound that the kernels tighten from their own candidates.
+Winners, rankings and FP64 scores are the oracle's, bit for bit."""
+import math
+
+import pytest
+
+import episdet
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(3, 1, 1), (4, 31, 1100), (33, 1024, 1025), (64, 700, 3000), (65, 2049, 2048), (98, 40, 25)]
+
+
+@pytest.mark.parametrize("n,Nc,Nt", SIZES)
+@pytest.mark.parametrize("score", [episdet.K2, episdet.MI])
+def test_unit_edges(n, Nc, Nt, score):
+    syn = episdet.generate(n, Nc, Nt, seed=300 + n, planted_sets=1 if n >= 64 else 0)
+    ref_p, ref_s = O.ranked(syn.cases, syn.controls, Nc, Nt, 3, score)
+    with episdet.Dataset.from_synthetic(syn) as ds:
+        for tile in (3, 4, 5):
+            print(f"edges n={n} Nc={Nc} Nt={Nt} score={score} tile={tile}", flush=True)
+            r = ds.run(3, score, path=episdet.PATH_FUSED_MFMA, tile=tile)
+            assert r["packed"] == int(ref_p[0]) and r["best_score"] == float(ref_s[0])
+            for k in (2, 65, 1024):
+                p, s, _ = ds.topk(3, k, score=score, path=episdet.PATH_FUSED_MFMA, tile=tile)
+                m = min(k, math.comb(n, 3))
+                assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
