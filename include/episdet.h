@@ -149,8 +149,8 @@ typedef struct {
                                    hipEvents on the launching stream             */
     double rescore_ms;          /* device time of the FP64 re-scoring            */
     double prep_ms;             /* host time of single/pair table builds in this
-                                   call (0 when cached); the single counts are
-                                   recomputed without a wait of their own, so
+                                   call (0 when cached); they are rebuilt on the
+                                   search's stream with no wait of their own, so
                                    their device time falls in the search's      */
     double wall_s;              /* host wall-clock of this call                  */
     double fp32_max_abs_err;    /* max |FP32 - FP64| over re-scored candidates   */
@@ -160,7 +160,8 @@ typedef struct {
                                    rerun the search in windows                  */
     int tile;                   /* kernel tile id used                           */
     int seeded;                 /* 3-way fused: 1 if the search started from a
-                                   bound found through the best pairs          */
+                                   bound found through the best pairs (top-k
+                                   too, unless candidate_cap is set)           */
     int reserved[5];
 } episdet_result;
 
@@ -181,7 +182,7 @@ int episdet_run(episdet_dataset *ds, const episdet_options *opt, episdet_result 
  *    samples);
  *  - PLAIN, rebuild and autotune are refused (EPISDET_ERR_INVALID): they
  *    allocate buffers of their own;
- *  - no seeding pre-pass (result.seeded = 0): it runs a search of its own.
+ *  - no seeding from the best pairs (result.seeded = 0).
  * Calls share the array of their device, which keeps the last call's
  * contents, so calls that overlapped on one device would race: the library
  * runs the calls of a process one at a time (one lock).  Dataset creation

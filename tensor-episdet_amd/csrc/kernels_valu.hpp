@@ -950,79 +950,149 @@ struct RescoreArgs {
     uint32_t *out_cells;                // [count][2][3^k], may be null
 };
 
-// One wave per set: counts the 2^k AND-cells of both classes straight from
-// the planes, derives every cell, scores in FP64.
-__device__ __forceinline__ void rescore_one(const RescoreArgs &p, int i)
+// The 2^k AND-counts of a set over one class by one wave; every lane returns
+// all of them.  Rows are whole 128-byte lines, four words a lane and step.
+template <int ORDER>
+__device__ __forceinline__ void wave_counts(const uint32_t *base, int W, const int (&s)[3], int lane, uint32_t (&n8)[8])
 {
-    const int lane = threadIdx.x;
-    const unsigned long long pk = p.cand[i];
-    int s[3];
-    if (p.order == 3) {
-        s[0] = (int)(pk & 0x1FFFFF);
-        s[1] = (int)((pk >> 21) & 0x1FFFFF);
-        s[2] = (int)((pk >> 42) & 0x1FFFFF);
-    } else {
-        s[0] = (int)(pk & 0xFFFFFFFFu);
-        s[1] = (int)(pk >> 32);
-        s[2] = 0;
-    }
-    uint32_t n8[2][8];
-    for (int cls = 0; cls < 2; cls++) {
-        const uint32_t *base = cls ? p.p1 : p.p0;
-        const int W = cls ? p.W1 : p.W0;
-        uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        const uint32_t *r0 = base + (size_t)s[0] * 2 * W, *r1 = base + (size_t)s[1] * 2 * W;
-        const uint32_t *r2 = base + (size_t)s[2] * 2 * W;
-        for (int w = lane; w < W; w += 64) {
-            if (p.order == 3) {
+    uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const uint32_t *r[3];
 #pragma unroll
-                for (int x = 0; x < 2; x++)
+    for (int o = 0; o < 3; o++) r[o] = base + (size_t)s[o] * 2 * W;
+    for (int w = lane * 4; w < W; w += 256) {
+        uint4 v[ORDER][2];
 #pragma unroll
-                    for (int y = 0; y < 2; y++)
+        for (int o = 0; o < ORDER; o++)
 #pragma unroll
-                        for (int z = 0; z < 2; z++)
-                            c[x * 4 + y * 2 + z] += __popc(r0[x * W + w] & r1[y * W + w] & r2[z * W + w]);
-            } else {
+            for (int k = 0; k < 2; k++) v[o][k] = *(const uint4 *)(r[o] + (size_t)k * W + w);
+        const auto pop4 = [](const uint4 &q) { return __popc(q.x) + __popc(q.y) + __popc(q.z) + __popc(q.w); };
+        const auto and4 = [](const uint4 &p, const uint4 &q) {
+            return make_uint4(p.x & q.x, p.y & q.y, p.z & q.z, p.w & q.w);
+        };
 #pragma unroll
-                for (int x = 0; x < 2; x++)
+        for (int x = 0; x < 2; x++)
 #pragma unroll
-                    for (int y = 0; y < 2; y++) c[x * 2 + y] += __popc(r0[x * W + w] & r1[y * W + w]);
+            for (int y = 0; y < 2; y++) {
+                const uint4 xy = and4(v[0][x], v[1][y]);
+                if constexpr (ORDER == 3) {
+                    c[x * 4 + y * 2] += pop4(and4(xy, v[2][0]));
+                    c[x * 4 + y * 2 + 1] += pop4(and4(xy, v[2][1]));
+                } else {
+                    c[x * 2 + y] += pop4(xy);
+                }
             }
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) n8[cls][k] = wave_sum_u(c[k]);
     }
-    if (lane != 0) return;
-    uint32_t cas[27], ctl[27];
-    int nc;
-    if (p.order == 3) {
-        nc = 27;
-        const Singles sx = ld_global(p.singles, s[0]), sy = ld_global(p.singles, s[1]), sz = ld_global(p.singles, s[2]);
+#pragma unroll
+    for (int k = 0; k < (1 << ORDER); k++) n8[k] = wave_sum_u(c[k]);
+}
+
+// Both classes' cells of one set (uniform over the wave), in every lane.
+template <int ORDER, int NC>
+__device__ __forceinline__ void wave_cells(const RescoreArgs &p, const int (&s)[3], int lane, uint32_t (&cas)[NC],
+                                           uint32_t (&ctl)[NC])
+{
+    uint32_t nc8[8], nt8[8];
+    wave_counts<ORDER>(p.p0, p.W0, s, lane, nc8);
+    wave_counts<ORDER>(p.p1, p.W1, s, lane, nt8);
+    const Singles sx = ld_global(p.singles, s[0]), sy = ld_global(p.singles, s[1]);
+    if constexpr (ORDER == 3) {
+        const Singles sz = ld_global(p.singles, s[2]);
         uint32_t xy[9], xz[9], yz[9];
         pair9_lookup(p.pairs, p.n, sx, sy, s[0], s[1], 0, (uint32_t)p.N0, xy);
         pair9_lookup(p.pairs, p.n, sx, sz, s[0], s[2], 0, (uint32_t)p.N0, xz);
         pair9_lookup(p.pairs, p.n, sy, sz, s[1], s[2], 0, (uint32_t)p.N0, yz);
-        triplet27(n8[0], xy, xz, yz, cas);
+        triplet27(nc8, xy, xz, yz, cas);
         pair9_lookup(p.pairs, p.n, sx, sy, s[0], s[1], 1, (uint32_t)p.N1, xy);
         pair9_lookup(p.pairs, p.n, sx, sz, s[0], s[2], 1, (uint32_t)p.N1, xz);
         pair9_lookup(p.pairs, p.n, sy, sz, s[1], s[2], 1, (uint32_t)p.N1, yz);
-        triplet27(n8[1], xy, xz, yz, ctl);
+        triplet27(nt8, xy, xz, yz, ctl);
     } else {
-        nc = 9;
-        const Singles sa = ld_global(p.singles, s[0]), sb = ld_global(p.singles, s[1]);
-        pair9(n8[0][0], n8[0][1], n8[0][2], n8[0][3], sa.x, sa.y, sb.x, sb.y, (uint32_t)p.N0, cas);
-        pair9(n8[1][0], n8[1][1], n8[1][2], n8[1][3], sa.z, sa.w, sb.z, sb.w, (uint32_t)p.N1, ctl);
+        pair9(nc8[0], nc8[1], nc8[2], nc8[3], sx.x, sx.y, sy.x, sy.y, (uint32_t)p.N0, cas);
+        pair9(nt8[0], nt8[1], nt8[2], nt8[3], sx.z, sx.w, sy.z, sy.w, (uint32_t)p.N1, ctl);
     }
+}
+
+__device__ __forceinline__ double shfl_d(double v, int src)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, src);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), src);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// k2_f64 / mi_f64 by one wave that holds the cells in every lane: lane c
+// looks cell c's table entries up, and the terms are added in the order of
+// the cells, the same operations on the same values, so the scores agree bit
+// for bit.  One lane doing the 81 dependent lookups took most of the 7 to 12
+// us that re-scoring a handful of candidates cost.
+template <int NC>
+__device__ __forceinline__ double wave_score_f64(const RescoreArgs &p, const uint32_t (&cas)[NC],
+                                                 const uint32_t (&ctl)[NC], int lane)
+{
+#pragma clang fp contract(off)
+    if (!cells_valid(cas, ctl, NC, p.N0, p.N1)) return __builtin_nan("");
+    uint32_t a = 0, b = 0;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        a = lane == c ? cas[c] : a;
+        b = lane == c ? ctl[c] : b;
+    }
+    const double *T = p.t64;
+    if (p.score == SCORE_K2) {
+        double t = T[b] + T[a];
+        t = t - T[b + a + 1];
+        double s = 0.0;
+#pragma unroll
+        for (int c = 0; c < NC; c++) s = s + shfl_d(t, c);
+        return fabs(s);
+    }
+    const double invN = 1.0 / (double)(p.N0 + p.N1);
+    double hY = -((double)p.N0 * invN) * T[p.N0];
+    hY = hY - ((double)p.N1 * invN) * T[p.N1];
+    const double pc = (double)a * invN, pt = (double)b * invN;
+    const double qa = pc * T[a], qb = pt * T[b], qn = (pc + pt) * T[a + b];
+    double hG = 0.0, hGY = 0.0;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        hGY = hGY - shfl_d(qa, c);
+        hGY = hGY - shfl_d(qb, c);
+        hG = hG - shfl_d(qn, c);
+    }
+    return (hG + hY) - hGY;
+}
+
+// One wave per set: counts the 2^k AND-cells of both classes straight from
+// the planes, derives every cell, scores in FP64 (returned in every lane).
+template <int ORDER, int NC>
+__device__ __forceinline__ double rescore_set(const RescoreArgs &p, unsigned long long pk, int i, int lane)
+{
+    int s[3];
+    s[0] = uniform((int)(ORDER == 3 ? pk & 0x1FFFFF : pk & 0xFFFFFFFFu));
+    s[1] = uniform((int)(ORDER == 3 ? (pk >> 21) & 0x1FFFFF : pk >> 32));
+    s[2] = uniform((int)(ORDER == 3 ? (pk >> 42) & 0x1FFFFF : 0));
+    uint32_t cas[NC], ctl[NC];
+    wave_cells<ORDER, NC>(p, s, lane, cas, ctl);
     if (p.out_cells) {
-        uint32_t *o = p.out_cells + (size_t)i * 2 * nc;
-        for (int c = 0; c < nc; c++) {
-            o[c] = cas[c];
-            o[nc + c] = ctl[c];
-        }
+        uint32_t *o = p.out_cells + (size_t)i * 2 * NC;
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+            if (lane == c) {
+                o[c] = cas[c];
+                o[NC + c] = ctl[c];
+            }
     }
-    if (p.out_s64)
-        p.out_s64[i] =
-            p.score == SCORE_K2 ? k2_f64(cas, ctl, nc, p.N0, p.N1, p.t64) : mi_f64(cas, ctl, nc, p.N0, p.N1, p.t64);
+    double v = 0.0;
+    if (p.out_s64) {
+        v = wave_score_f64<NC>(p, cas, ctl, lane);
+        if (lane == 0) p.out_s64[i] = v;
+    }
+    return v;
+}
+__device__ __forceinline__ double rescore_one(const RescoreArgs &p, int i)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned long long pk = p.cand[i];
+    return p.order == 3 ? rescore_set<3, 27>(p, pk, i, lane) : rescore_set<2, 9>(p, pk, i, lane);
 }
 
 __global__ __launch_bounds__(64) void k_rescore(RescoreArgs p)
@@ -1054,12 +1124,11 @@ __global__ __launch_bounds__(64) void k_rescore_after(RescoreArgs p, const unsig
     }
     if (over || count > cap) return;
     for (unsigned i = blockIdx.x; i < count; i += gridDim.x) {
-        rescore_one(p, (int)i);
-        // lane 0 wrote the FP64 score of set i just now
+        const double v = rescore_one(p, (int)i);
         if (threadIdx.x == 0 && i < hs.slots) {
             hs.packed[i] = p.cand[i];
             hs.s32[i] = cand_s32[i];
-            hs.s64[i] = p.out_s64[i];
+            hs.s64[i] = v;
         }
     }
 }
@@ -1173,23 +1242,92 @@ __global__ void k_term_error(int score, int N, float invN, float k0, float c32, 
     if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(e));
 }
 
-// Small fill kernels (no hipMemsetAsync, so the sequence stays capturable).
-// queue0: first work unit; best0: starting global bound (key), 0 for +inf.
-// queue[0] is the work queue, queue[QLINE (1 + x)] the per-XCD queues (fetch_xcd):
-// all start at unit queue0.
-__global__ void k_init_search(unsigned long long *queue, unsigned *best_key, unsigned *cand_count,
-                              unsigned long long *best_key64, unsigned long long *checksum,
-                              unsigned long long queue0, unsigned best0)
+// Resets a search's control words: queue0 the first work unit, best0 the
+// starting global bound (key; 0: +inf).  queue[0] is the work queue,
+// queue[QLINE (1 + x)] the per-XCD queues (fetch_xcd): all start at unit queue0.
+struct InitArgs {
+    unsigned long long *queue;
+    unsigned *best_key, *cand_count;
+    unsigned long long *best_key64, *checksum, queue0;
+    unsigned best0;
+};
+__device__ __forceinline__ void init_search(const InitArgs &a)
+{
+    *a.queue = a.queue0;
+    for (unsigned x = 0; x < 8; x++) a.queue[QLINE * (1 + x)] = a.queue0 > x ? (a.queue0 - x + 7) / 8 : 0ull;
+    *a.best_key = a.best0 ? a.best0 : 0xFF800000u; // key of +inf
+    a.cand_count[0] = 0u;
+    a.cand_count[1] = 0u;                          // overflow flag
+    *a.best_key64 = 0xFFF0000000000000ull;         // key of +inf (double)
+    *a.checksum = 0ull;
+}
+// Resets them, and writes the search's argument block (a job of one, units
+// [0, units)) to its slot in device memory: the block travels as a kernel argument, so
+// no host buffer has to outlive the call and nothing waits for a copy.
+template <typename A>
+__global__ void k_init_args(InitArgs ia, A args, A *slot, unsigned long long *job_start, unsigned long long units)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *queue = queue0;
-        for (unsigned x = 0; x < 8; x++) queue[QLINE * (1 + x)] = queue0 > x ? (queue0 - x + 7) / 8 : 0ull;
-        *best_key = best0 ? best0 : 0xFF800000u; // key of +inf
-        cand_count[0] = 0u;
-        cand_count[1] = 0u;                      // overflow flag
-        *best_key64 = 0xFFF0000000000000ull;     // key of +inf (double)
-        *checksum = 0ull;
+        init_search(ia);
+        *slot = args;
+        job_start[0] = 0ull;
+        job_start[1] = units;
     }
+}
+
+// Units of the 3-way group (Y tile ty, Z tile tz): the X values some set of it
+// needs, xstep per unit; 0 if it holds no X < Y < Z.
+__host__ __device__ inline int group_units(int n, int TY, int TZ, int xstep, int ty, int tz)
+{
+    const int ylo = ty * TY, yhi = (ylo + TY < n ? ylo + TY : n) - 1;
+    const int zhi = (tz * TZ + TZ < n ? tz * TZ + TZ : n) - 1;
+    if (zhi <= ylo) return 0;
+    const int x = yhi < zhi - 1 ? yhi : zhi - 1;
+    return x > 0 ? (x + xstep - 1) / xstep : 0;
+}
+
+// The 3-way groups that hold a set, in (ty, tz) order, and the first unit of
+// each (gstart[ngroups]: all units).  One workgroup; a thread lists the groups
+// of a row ty, after a scan over the rows of a turn.
+__global__ __launch_bounds__(1024) void k_groups(int n, int TY, int TZ, int xstep, int2 *groups,
+                                                 unsigned long long *gstart)
+{
+    __shared__ unsigned long long su[1024], sg[1024];
+    const int nty = (n + TY - 1) / TY, ntz = (n + TZ - 1) / TZ, t = threadIdx.x;
+    unsigned long long u0 = 0, g0 = 0;
+    for (int r0 = 0; r0 < nty; r0 += 1024) {
+        const int ty = r0 + t, tz0 = (int)((long long)ty * TY / TZ);
+        unsigned long long u = 0, g = 0;
+        if (ty < nty)
+            for (int tz = tz0; tz < ntz; tz++) {
+                const int k = group_units(n, TY, TZ, xstep, ty, tz);
+                u += (unsigned)k;
+                g += k > 0;
+            }
+        su[t] = u;
+        sg[t] = g;
+        __syncthreads();
+        for (int o = 1; o < 1024; o <<= 1) {
+            const unsigned long long pu = t >= o ? su[t - o] : 0ull, pg = t >= o ? sg[t - o] : 0ull;
+            __syncthreads();
+            su[t] += pu;
+            sg[t] += pg;
+            __syncthreads();
+        }
+        unsigned long long at = u0 + su[t] - u, gi = g0 + sg[t] - g;
+        if (ty < nty)
+            for (int tz = tz0; tz < ntz; tz++) {
+                const int k = group_units(n, TY, TZ, xstep, ty, tz);
+                if (k <= 0) continue;
+                groups[gi] = make_int2(ty, tz);
+                gstart[gi++] = at;
+                at += (unsigned)k;
+            }
+        u0 += su[1023];
+        g0 += sg[1023];
+        __syncthreads();
+    }
+    if (t == 0) gstart[g0] = u0;
 }
 
 }  // namespace episdet

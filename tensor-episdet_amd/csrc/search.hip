@@ -29,6 +29,7 @@
 #include "kernels_mfma4.hpp"
 #include "kernels_mfma_pairs2.hpp"
 #include "kernels_mfma5.hpp"
+#include "kernels_seed.hpp"
 
 using namespace episdet;
 
@@ -36,6 +37,7 @@ namespace {
 
 constexpr int BLOCK = 256;            // the reference's BLOCK_SIZE (Makefile:2)
 constexpr int PLAIN_GROUP = 16;       // 3-way rounds per FP4 count launch of the plain path
+constexpr size_t SEED_WORDS = 2 * SEED_BLOCKS + SEED_MAX_PAIRS;   // block bests, picked pairs
 constexpr int PLAIN_GROUP2 = 32;      // 2-way rounds per FP4 count launch of the plain path
 // Words per plane row on the device: the samples rounded up to 1024 (the
 // reference's own padding), a whole chunk of every kernel that stages
@@ -185,7 +187,10 @@ struct episdet_dataset {
     int cu = 0;
     void *jobargs = nullptr;                  // device copy of one kernel argument block
     unsigned long long *jobstart = nullptr;   // {0, units} for a batch of one
-    std::vector<unsigned char> args_sent;     // what jobargs / jobstart last received (upload_single)
+    unsigned long long *gstart = nullptr;     // 3-way work-unit groups (k_groups), and the tile they are for
+    int2 *groups = nullptr;
+    int group_tile[3] = {0, 0, 0};            // TY, TZ, X per unit; 0: none yet
+    unsigned long long *seed = nullptr;       // best pairs of the seeding kernels (SEED_WORDS)
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};   // search start / end, re-score end
     unsigned char *stage = nullptr;           // pinned, device-mapped: candidate count + the first candidates
     unsigned char *stage_dev = nullptr;       // the device's address of `stage`
@@ -546,38 +551,33 @@ void launch_tri_mfma(int tile, int blocks, const BatchTri &bt, hipStream_t s)
 
 static_assert(sizeof(TriArgs) <= 1024 && sizeof(PairArgs) <= 1024, "argument slot too small");
 
-// Copies one argument block to the dataset's device slot, for a batch of one.
-// The kernels only read the slot, so a block identical to the last one sent
-// is not sent again (repeated searches of one dataset skip the copies and
-// their synchronisation).  Inside a no-allocation call the slot is in the
-// shared scratch array, which other datasets' calls overwrite: always sent.
-template <typename A>
-int upload_single(episdet_dataset *ds, const A &a, unsigned long long units)
+InitArgs init_args(const episdet_dataset *ds, unsigned long long u0 = 0, unsigned seed_key = 0)
 {
-    const unsigned long long js[2] = {0ull, units};
-    unsigned char key[sizeof(A) + sizeof js];
-    std::memcpy(key, &a, sizeof(A));
-    std::memcpy(key + sizeof(A), js, sizeof js);
-    if (!t_scr && ds->args_sent.size() == sizeof key && std::memcmp(ds->args_sent.data(), key, sizeof key) == 0)
-        return EPISDET_OK;
-    ds->args_sent.clear();
-    HIPCHK(hipMemcpyAsync(ds->jobargs, &a, sizeof(A), hipMemcpyHostToDevice, ds->stream));
-    HIPCHK(hipMemcpyAsync(ds->jobstart, js, sizeof js, hipMemcpyHostToDevice, ds->stream));
-    HIPCHK(hipStreamSynchronize(ds->stream));
-    if (!t_scr) ds->args_sent.assign(key, key + sizeof key);
+    return InitArgs{ds->ctl->queue,      &ds->ctl->best32, &ds->ctl->cand_count, &ds->ctl->best64,
+                    &ds->ctl->checksum, u0,               seed_key};
+}
+
+// Resets the dataset's control block on its stream (queue at u0, global
+// bound at seed_key, 0: +inf; no candidates) and writes a kernel's argument
+// block to the dataset's slot, for a batch of one.
+template <typename A>
+int init_single(episdet_dataset *ds, const A &a, unsigned long long units, unsigned long long u0 = 0,
+                unsigned seed_key = 0)
+{
+    hipLaunchKernelGGL((k_init_args<A>), dim3(1), dim3(64), 0, ds->stream, init_args(ds, u0, seed_key), a,
+                       (A *)ds->jobargs, ds->jobstart, units);
+    HIPCHK(hipGetLastError());
     return EPISDET_OK;
 }
 
-// upload = false: the caller has already copied `a` to the dataset's
-// argument slot (upload_single), e.g. before recording a timing event.
+// The caller has written `a` to the dataset's argument slot (init_single).
 template <int MODE>
-int dispatch_tri_mfma(episdet_dataset *ds, int tile, TriArgs &a, hipStream_t s, bool upload = true)
+int dispatch_tri_mfma(episdet_dataset *ds, int tile, TriArgs &a, hipStream_t s)
 {
     const void *k = mfma_kernel<MODE>(tile);
     int per = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, mfma_threads(tile), 0) != hipSuccess || per < 1)
         per = 1;
-    if (upload) CHK(upload_single(ds, a, a.nunits));
     BatchTri bt;
     bt.jobs = (const TriArgs *)ds->jobargs;
     bt.job_start = ds->jobstart;
@@ -649,9 +649,8 @@ int launch_pairs_mfma(int tile, int blocks, const BatchPair &bp, hipStream_t s)
 void fill_pairs(episdet_dataset *ds, PairArgs &a, bool mfma, int tile);
 
 template <int MODE>
-int dispatch_pairs(episdet_dataset *ds, bool mfma, int tile, PairArgs &a, hipStream_t s, bool upload = true)
+int dispatch_pairs(episdet_dataset *ds, bool mfma, int tile, PairArgs &a, hipStream_t s)
 {
-    if (upload) CHK(upload_single(ds, a, a.nunits));
     BatchPair bp;
     bp.jobs = (const PairArgs *)ds->jobargs;
     bp.job_start = ds->jobstart;
@@ -679,18 +678,14 @@ void build_groups(int n, int TY, int TZ, std::vector<int2> &groups, std::vector<
     gstart.clear();
     unsigned long long acc = 0;
     const int nty = (n + TY - 1) / TY, ntz = (n + TZ - 1) / TZ;
-    for (int ty = 0; ty < nty; ty++) {
-        const int ylo = ty * TY, yhi = std::min(ylo + TY, n) - 1;
+    for (int ty = 0; ty < nty; ty++)
         for (int tz = 0; tz < ntz; tz++) {
-            const int zhi = std::min(tz * TZ + TZ, n) - 1;
-            if (zhi <= ylo) continue;
-            const int xcount = std::min(yhi, zhi - 1);
-            if (xcount <= 0) continue;
+            const int units = group_units(n, TY, TZ, xstep, ty, tz);
+            if (units <= 0) continue;
             groups.push_back(make_int2(ty, tz));
             gstart.push_back(acc);
-            acc += (unsigned long long)((xcount + xstep - 1) / xstep);
+            acc += (unsigned long long)units;
         }
-    }
     gstart.push_back(acc);
 }
 
@@ -756,20 +751,10 @@ void fill_pairs(episdet_dataset *ds, PairArgs &a, bool mfma, int tile)
     }
 }
 
-// Resets the dataset's control block on its stream: queue at u0, global
-// bound at seed_key (0: +inf), no candidates.  Both values travel as kernel
-// arguments, so no host memory has to outlive the call.
-int init_ctl(episdet_dataset *ds, unsigned long long u0 = 0, unsigned seed_key = 0)
-{
-    hipLaunchKernelGGL(k_init_search, dim3(1), dim3(64), 0, ds->stream, ds->ctl->queue, &ds->ctl->best32,
-                       &ds->ctl->cand_count, &ds->ctl->best64, &ds->ctl->checksum, u0, seed_key);
-    HIPCHK(hipGetLastError());
-    return EPISDET_OK;
-}
-
 // The 3-way pair table, built once per dataset; rebuild = true builds it
 // again in place (the planes never change, so this only makes the build
-// part of a call's cost).
+// part of a call's cost).  Not waited for: what follows on the dataset's
+// stream reads it.
 int ensure_pairs(episdet_dataset *ds, bool rebuild)
 {
     if (ds->pairs && !rebuild) return EPISDET_OK;
@@ -783,14 +768,12 @@ int ensure_pairs(episdet_dataset *ds, bool rebuild)
         ds->pairs = nullptr;
         return EPISDET_ERR_ALLOC;
     }
-    CHK(init_ctl(ds));
     PairArgs a;
     const bool mfma = mfma_ok(ds);
     fill_pairs(ds, a, mfma, 0);
     a.pairs = ds->pairs;
-    CHK(dispatch_pairs<MODE_PAIRTABLE>(ds, mfma, 0, a, ds->stream));
-    HIPCHK(hipStreamSynchronize(ds->stream));
-    return EPISDET_OK;
+    CHK(init_single(ds, a, a.nunits));
+    return dispatch_pairs<MODE_PAIRTABLE>(ds, mfma, 0, a, ds->stream);
 }
 
 inline bool better(int score, double s, unsigned long long p, double bs, unsigned long long bp)
@@ -961,31 +944,58 @@ int collect_best(episdet_dataset *ds, int order, int score, int count, episdet_r
 }
 
 // One fused kernel configuration for one dataset and search: the argument
-// block and, for 3-way, the work-unit groups (host copy kept for counting
-// the sets of a unit window).
+// block; the 3-way work-unit groups are the dataset's (ensure_groups).
 struct FusedPlan {
     int order = 0, score = 0, path = 0, tile = 0;
     bool mfma = false;
     TriArgs ta{};
     PairArgs pa{};
     ScoreCtx sc{};
-    std::vector<int2> groups;
-    std::vector<unsigned long long> gstart;
-    unsigned long long *d_gstart = nullptr;
-    int2 *d_groups = nullptr;
     unsigned long long nunits = 0;
-    unsigned seed_key = 0;       // starting global bound (best32), 0: none (see seed_from_pairs)
-    bool own_groups = false;     // d_gstart / d_groups allocated here (not in `scratch`)
-    FusedPlan() = default;
-    FusedPlan(const FusedPlan &) = delete;
-    FusedPlan &operator=(const FusedPlan &) = delete;
-    ~FusedPlan()
+    unsigned seed_key = 0;       // starting global bound (best32), 0: none
+    int seed_pairs = 0;          // 3-way: > 0: the launch starts from the triplets of this many best pairs
+    void group_tile(int (&t)[3]) const
     {
-        if (!own_groups) return;
-        if (d_gstart) (void)hipFree(d_gstart);
-        if (d_groups) (void)hipFree(d_groups);
+        t[0] = mfma ? mfma_ty(tile) : 16 * TRI_TILES[tile].A;
+        t[1] = mfma ? mfma_tz(tile) : 16 * TRI_TILES[tile].B;
+        t[2] = mfma ? mfma_xstep(tile) : 1;
     }
 };
+
+// The 3-way work-unit groups of a tile in the dataset's buffers, listed on
+// its stream; kept while searches use the same tile.  *ngroups and *nunits: their
+// numbers.  Every tile is at least 32 x 32, which sizes the buffers.
+int ensure_groups(episdet_dataset *ds, const int (&t)[3], int *ngroups, unsigned long long *nunits)
+{
+    const size_t side = ((size_t)ds->n + 31) / 32, most = side * (side + 1) / 2;
+    if (!t_scr && !ds->gstart) {
+        if (dev_malloc((void **)&ds->gstart, sizeof(unsigned long long) * (most + 1)) != hipSuccess ||
+            dev_malloc((void **)&ds->groups, sizeof(int2) * most) != hipSuccess) {
+            if (ds->gstart) (void)hipFree(ds->gstart);
+            ds->gstart = nullptr;
+            ds->groups = nullptr;
+            return EPISDET_ERR_ALLOC;
+        }
+    }
+    const int nty = (ds->n + t[0] - 1) / t[0], ntz = (ds->n + t[1] - 1) / t[1];
+    size_t g = 0;
+    unsigned long long u = 0;
+    for (int ty = 0; ty < nty; ty++)
+        for (int tz = (int)((long long)ty * t[0] / t[1]); tz < ntz; tz++) {
+            const int k = group_units(ds->n, t[0], t[1], t[2], ty, tz);
+            u += (unsigned long long)k;
+            g += k > 0;
+        }
+    if (g == 0) return EPISDET_ERR_INVALID;
+    if (g > most || (t_scr && g > t_scr->max_groups)) return EPISDET_ERR_INTERNAL;
+    *ngroups = (int)g;
+    *nunits = u;
+    if (!t_scr && std::memcmp(ds->group_tile, t, sizeof t) == 0) return EPISDET_OK;
+    hipLaunchKernelGGL(k_groups, dim3(1), dim3(1024), 0, ds->stream, ds->n, t[0], t[1], t[2], ds->groups, ds->gstart);
+    HIPCHK(hipGetLastError());
+    if (!t_scr) std::memcpy(ds->group_tile, t, sizeof t);
+    return EPISDET_OK;
+}
 
 bool tile_valid(int order, int path, int tile)
 {
@@ -1007,33 +1017,14 @@ int plan_fused(episdet_dataset *ds, int order, int score, int path, int tile, Fu
     if (!tile_valid(order, path, tile)) return EPISDET_ERR_INVALID;
     pl.sc = make_ctx(ds, score, order);
     if (order == 3) {
-        if (pl.mfma) {
-            build_groups(ds->n, mfma_ty(tile), mfma_tz(tile), pl.groups, pl.gstart, mfma_xstep(tile));
-        } else {
-            const Tri3Tile t = TRI_TILES[tile];
-            build_groups(ds->n, 16 * t.A, 16 * t.B, pl.groups, pl.gstart);
-        }
-        if (pl.groups.empty()) return EPISDET_ERR_INVALID;
-        if (t_scr) {
-            if (pl.groups.size() > t_scr->max_groups) return EPISDET_ERR_INTERNAL;   // sized by the caller
-            pl.d_gstart = t_scr->gstart;
-            pl.d_groups = t_scr->groups;
-        } else {
-            pl.own_groups = true;
-            if (dev_malloc((void **)&pl.d_gstart, sizeof(unsigned long long) * pl.gstart.size()) != hipSuccess)
-                return EPISDET_ERR_ALLOC;
-            if (dev_malloc((void **)&pl.d_groups, sizeof(int2) * pl.groups.size()) != hipSuccess)
-                return EPISDET_ERR_ALLOC;
-        }
-        HIPCHK(hipMemcpy(pl.d_gstart, pl.gstart.data(), sizeof(unsigned long long) * pl.gstart.size(),
-                         hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(pl.d_groups, pl.groups.data(), sizeof(int2) * pl.groups.size(), hipMemcpyHostToDevice));
+        int t[3], ngroups = 0;
+        pl.group_tile(t);
+        CHK(ensure_groups(ds, t, &ngroups, &pl.nunits));
         fill_tri_common(ds, pl.ta);
         pl.ta.sc = pl.sc;
-        pl.ta.gstart = pl.d_gstart;
-        pl.ta.groups = pl.d_groups;
-        pl.ta.ngroups = (int)pl.groups.size();
-        pl.nunits = pl.gstart.back();
+        pl.ta.gstart = ds->gstart;
+        pl.ta.groups = ds->groups;
+        pl.ta.ngroups = ngroups;
         pl.ta.nunits = pl.nunits;
     } else {
         fill_pairs(ds, pl.pa, pl.mfma, tile);
@@ -1054,6 +1045,53 @@ unsigned long long unit_sets_max(const FusedPlan &pl)
     }
     if (pl.mfma) return pl.tile == 0 ? (unsigned long long)P2_TA * P2_TB : (unsigned long long)P3_TA * P3_TB;
     return 256ull * PAIR_TILES[pl.tile] * PAIR_TILES[pl.tile];
+}
+
+// A starting global bound for a 3-way search, on its stream between the reset
+// of the control block and the search (kernels_seed.hpp): the best FP32
+// badness among the triplets that contain one of the best pairs, or for top-k
+// the k-th best.  Some sets reach it, as they reach the minimum a workgroup
+// publishes, so the winner, the k best and every set tied with them still
+// become candidates; the score bounds then skip FP32 scores from the first unit on when
+// strongly associated triplets have associated pairs.
+constexpr int SEED_PAIRS = 4;
+int seed_from_pairs(episdet_dataset *ds, const FusedPlan &pl, int topk)
+{
+    SeedArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.r = rescore_args(ds, 3, pl.score);
+    a.r.cand = nullptr;
+    a.r.out_s64 = nullptr;
+    a.sc = pl.sc;
+    a.blk = ds->seed;
+    a.pick = ds->seed + 2 * SEED_BLOCKS;
+    a.blocks = std::min(SEED_BLOCKS, ds->n - 1);
+    a.npairs = pl.seed_pairs;
+    a.best_key = &ds->ctl->best32;
+    a.s32 = topk ? ds->cand_s32 : nullptr;     // free until the search appends
+    const int m = a.npairs * ds->n;
+    hipLaunchKernelGGL(k_seed_pairs, dim3(a.blocks), dim3(256), 0, ds->stream, a);
+    hipLaunchKernelGGL(k_seed_pick, dim3(1), dim3(SEED_BLOCKS), 0, ds->stream, a);
+    hipLaunchKernelGGL(k_seed_triplets, dim3((m + 3) / 4), dim3(256), 0, ds->stream, a);
+    if (topk)
+        hipLaunchKernelGGL(k_seed_kth, dim3(1), dim3(1024), 0, ds->stream, ds->cand_s32, m, (unsigned)topk,
+                           &ds->ctl->best32);
+    HIPCHK(hipGetLastError());
+    return EPISDET_OK;
+}
+
+// Pairs whose triplets seed a 3-way search (0: none): 4 for the best set; for
+// the k best enough to hold about 2 k triplets, if those fit the candidate
+// slots they are kept in.  A no-allocation call goes without, and so does a
+// top-k search whose caller sets the candidate slots: those are chosen to
+// force the windowed rerun, whose windows start from exact scores.
+int seed_pairs(const episdet_dataset *ds, int topk, bool own_cap)
+{
+    if (t_scr || ds->n < 4) return 0;
+    if (!topk) return SEED_PAIRS;
+    if (own_cap) return 0;
+    const int p = std::min({std::max(SEED_PAIRS, (2 * topk + ds->n - 3) / (ds->n - 2)), SEED_MAX_PAIRS, ds->n - 1});
+    return (long long)p * ds->n <= (long long)ds->cand_cap ? p : 0;
 }
 
 // Issues the plan over work units [u0, u1) (the whole search is
@@ -1082,10 +1120,10 @@ int issue_fused(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned long long
     const bool mfma = pl.mfma;
     int rc = EPISDET_OK;
     // the batched kernels read their argument block from device memory (the
-    // VALU 3-way kernel takes it by value)
-    if (order == 3 && mfma) CHK(upload_single(ds, ta, ta.nunits));
-    else if (order == 2) CHK(upload_single(ds, pa, pa.nunits));
-    CHK(init_ctl(ds, u0, seed_key));
+    // VALU 3-way kernel takes it by value, and only finds a copy there)
+    if (order == 3) CHK(init_single(ds, ta, ta.nunits, u0, seed_key));
+    else CHK(init_single(ds, pa, pa.nunits, u0, seed_key));
+    if (pl.seed_pairs > 0) CHK(seed_from_pairs(ds, pl, topk));
     // the 3-way kernels that tighten the top-k bound from the candidates' own
     // scores (tighten_topk) must find +inf in slots not written yet
     if (topk && order == 3 && mfma && tile >= 3) {
@@ -1094,13 +1132,13 @@ int issue_fused(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned long long
     }
     HIPCHK(hipEventRecord(e0, ds->stream));
     if (topk)
-        rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_TOPK>(ds, tile, ta, ds->stream, false)
+        rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_TOPK>(ds, tile, ta, ds->stream)
                                 : dispatch_tri<MODE_TOPK>(ds, tile, ta, 0, ds->stream))
-                        : dispatch_pairs<MODE_TOPK>(ds, mfma, tile, pa, ds->stream, false);
+                        : dispatch_pairs<MODE_TOPK>(ds, mfma, tile, pa, ds->stream);
     else
-        rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_SEARCH>(ds, tile, ta, ds->stream, false)
+        rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_SEARCH>(ds, tile, ta, ds->stream)
                                 : dispatch_tri<MODE_SEARCH>(ds, tile, ta, 0, ds->stream))
-                        : dispatch_pairs<MODE_SEARCH>(ds, mfma, tile, pa, ds->stream, false);
+                        : dispatch_pairs<MODE_SEARCH>(ds, mfma, tile, pa, ds->stream);
     HIPCHK(hipEventRecord(e1, ds->stream));
     return rc;
 }
@@ -1166,64 +1204,6 @@ unsigned f2key_host(float f)
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// A starting global bound for a single-best 3-way search: the best exact
-// badness among the triplets that contain one of the SEED_PAIRS best pairs
-// (a 2-way top-k search of the same data), plus half the candidate margin.
-// Every FP32 badness is within that half margin of the exact one, so the set
-// that attains the seed scores at or below it in FP32: the seed is a bound
-// some set reaches, as a published block minimum would be, and the winner
-// and every set tied with it still become candidates.  With it the score
-// bounds skip FP32 scores from the first unit on when strongly associated
-// triplets have associated pairs; without such pairs it only costs the
-// pre-pass.  Returns false, leaving the search unseeded, on any failure.
-constexpr int SEED_PAIRS = 4;
-bool seed_from_pairs(episdet_dataset *ds, int score, float margin, unsigned *key)
-{
-    if (ds->n < 4) return false;
-    episdet_options o;
-    std::memset(&o, 0, sizeof o);
-    o.order = 2;
-    o.score = score;
-    o.path = EPISDET_PATH_AUTO;
-    unsigned long long pk[SEED_PAIRS];
-    double sc[SEED_PAIRS];
-    int cnt = 0;
-    episdet_result r;
-    if (episdet_run_topk(ds, &o, SEED_PAIRS, pk, sc, &cnt, &r) != EPISDET_OK || cnt < 1) return false;
-    std::vector<unsigned long long> sets;
-    sets.reserve((size_t)cnt * ds->n);
-    for (int i = 0; i < cnt && i < SEED_PAIRS; i++) {
-        const int a = (int)(pk[i] & 0xFFFFFFFFu), b = (int)(pk[i] >> 32);
-        for (int c = 0; c < ds->n; c++) {
-            if (c == a || c == b) continue;
-            int t[3] = {a, b, c};
-            std::sort(t, t + 3);
-            sets.push_back((unsigned long long)t[0] | ((unsigned long long)t[1] << 21) |
-                           ((unsigned long long)t[2] << 42));
-        }
-    }
-    if (sets.empty() || ensure_cand(ds, (unsigned)sets.size()) != EPISDET_OK) return false;
-    if (hipMemcpy(ds->cand, sets.data(), sizeof(unsigned long long) * sets.size(), hipMemcpyHostToDevice) !=
-        hipSuccess)
-        return false;
-    double ms = 0;
-    if (rescore(ds, 3, score, (int)sets.size(), &ms) != EPISDET_OK) return false;
-    std::vector<double> s64(sets.size());
-    if (hipMemcpy(s64.data(), ds->cand_s64, sizeof(double) * s64.size(), hipMemcpyDeviceToHost) != hipSuccess)
-        return false;
-    double best = INFINITY;
-    for (double v : s64) {
-        if (std::isnan(v)) return false;
-        best = std::min(best, score == EPISDET_SCORE_K2 ? v : -v);     // badness: lower is better
-    }
-    const double bound = best + 0.5 * (double)margin;
-    float f = (float)bound;
-    if ((double)f < bound) f = std::nextafter(f, INFINITY);
-    if (!std::isfinite(f)) return false;
-    *key = f2key_host(f);
-    return true;
-}
-
 // ------------------------------------------------------------ autotuner --
 //
 // For each shape (order, score, n, W0, W1) the tuner times every kernel
@@ -1280,12 +1260,15 @@ unsigned long long count_sets(const episdet_dataset *ds, const FusedPlan &pl, un
         const long long TY = pl.mfma ? mfma_ty(pl.tile) : 16 * TRI_TILES[pl.tile].A;
         const long long TZ = pl.mfma ? mfma_tz(pl.tile) : 16 * TRI_TILES[pl.tile].B;
         const long long XS = pl.mfma ? mfma_xstep(pl.tile) : 1;
-        size_t g = (size_t)(std::upper_bound(pl.gstart.begin(), pl.gstart.end(), u0) - pl.gstart.begin()) - 1;
+        std::vector<int2> groups;
+        std::vector<unsigned long long> gstart;
+        build_groups(ds->n, (int)TY, (int)TZ, groups, gstart, (int)XS);
+        size_t g = (size_t)(std::upper_bound(gstart.begin(), gstart.end(), u0) - gstart.begin()) - 1;
         for (unsigned long long u = u0; u < u1; u++) {
-            while (g + 1 < pl.groups.size() && pl.gstart[g + 1] <= u) g++;
-            const long long ylo = (long long)pl.groups[g].x * TY, zlo = (long long)pl.groups[g].y * TZ;
+            while (g + 1 < groups.size() && gstart[g + 1] <= u) g++;
+            const long long ylo = (long long)groups[g].x * TY, zlo = (long long)groups[g].y * TZ;
             const long long zhi = std::min(zlo + TZ, n);
-            for (long long X = XS * (long long)(u - pl.gstart[g]); X < XS * (long long)(u - pl.gstart[g] + 1); X++)
+            for (long long X = XS * (long long)(u - gstart[g]); X < XS * (long long)(u - gstart[g] + 1); X++)
                 for (long long Y = std::max(ylo, X + 1); Y < std::min(ylo + TY, n); Y++) {
                     const long long z0 = std::max(zlo, Y + 1);
                     if (zhi > z0) total += (unsigned long long)(zhi - z0);
@@ -1457,7 +1440,7 @@ int choose_kernel(episdet_dataset *ds, int order, int score, int *path, int *til
 // Key of the smallest float at or above badness + margin / 2, or 0 when
 // that is not finite.  A launch seeded with it keeps as candidates every set
 // whose exact badness is at or below `badness` (each FP32 badness is within
-// half the margin of the exact one), as seed_from_pairs argues.
+// half the margin of the exact one).
 unsigned seed_key_above(double badness, float margin)
 {
     const double bound = badness + 0.5 * (double)margin;
@@ -1539,13 +1522,8 @@ int run_fused(episdet_dataset *ds, const episdet_options *o, episdet_result *res
     if (t_scr) cap = std::min<unsigned long long>(cap, ds->cand_cap);
     CHK(ensure_cand(ds, (unsigned)cap));
     const ScoreCtx &sc = pl.sc;
-    // (the seeding pre-pass runs a top-k search with buffers of its own, so a
-    // no-allocation call goes without it: same winner, the bounds start later)
-    if (order == 3 && !topk && !t_scr) {
-        unsigned key = 0;
-        if (seed_from_pairs(ds, score, sc.margin, &key)) pl.seed_key = key;
-    }
-    res->seeded = pl.seed_key != 0;
+    if (order == 3) pl.seed_pairs = seed_pairs(ds, topk, o->candidate_cap > 0);
+    res->seeded = pl.seed_pairs > 0;
 
     Collected acc;
     acc.score = score;
@@ -1563,7 +1541,12 @@ int run_fused(episdet_dataset *ds, const episdet_options *o, episdet_result *res
             CHK(collect_host(stage_packed(ds->stage), stage_s32(ds->stage), stage_s64(ds->stage), count, acc));
         else CHK(collect(ds, count, acc));
     } else {
-        // more sets within the FP32 margin than slots: search again in windows
+        // more sets within the FP32 margin than slots: search again in
+        // windows, from the bound that the launch arrived at
+        Ctl end;
+        HIPCHK(hipMemcpy(&end, ds->ctl, sizeof end, hipMemcpyDeviceToHost));
+        pl.seed_pairs = 0;
+        if (end.best32 < 0xFF800000u) pl.seed_key = end.best32;
         CHK(run_sliced(ds, pl, topk, (unsigned)cap, hc, acc, &kms_total, &rms_total));
         res->fallback = 1;
     }
@@ -1622,10 +1605,14 @@ int run_plain(episdet_dataset *ds, const episdet_options *o, episdet_result *res
     TriArgs ta;
     if (order == 3) fill_tri_common(ds, ta);
     PairArgs pa{};
-    if (mfma && order == 3) CHK(upload_single(ds, ta, 0));    // the planes and sizes the count kernel reads
+    if (mfma && order == 3) {
+        CHK(init_single(ds, ta, 0));    // the planes and sizes the count kernel reads
+        HIPCHK(hipStreamSynchronize(ds->stream));   // it runs on other streams
+    }
     if (mfma && order == 2) {
         fill_pairs(ds, pa, true, 0);
-        CHK(upload_single(ds, pa, 0));
+        CHK(init_single(ds, pa, 0));
+        HIPCHK(hipStreamSynchronize(ds->stream));
     }
     PlainObjArgs po;
     std::memset(&po, 0, sizeof po);
@@ -1913,10 +1900,17 @@ int episdet_dataset_create(const unsigned *cases, const unsigned *controls, int 
     const unsigned *src[2] = {cases, controls};
     int rc = EPISDET_OK;
     if (hipStreamCreateWithFlags(&ds->stream, hipStreamNonBlocking) != hipSuccess) rc = EPISDET_ERR_HIP;
-    if (rc == EPISDET_OK && hipMalloc(&ds->ctl, sizeof(Ctl)) != hipSuccess) rc = EPISDET_ERR_ALLOC;
-    if (rc == EPISDET_OK && hipMalloc(&ds->jobargs, 1024) != hipSuccess) rc = EPISDET_ERR_ALLOC;
-    if (rc == EPISDET_OK && hipMalloc(&ds->jobstart, 2 * sizeof(unsigned long long)) != hipSuccess)
+    // control block, argument slot and the seeding kernels' pairs in one block
+    if (rc == EPISDET_OK && hipMalloc(&ds->ctl, sizeof(Ctl) + 1024 + 256 + sizeof(unsigned long long) * SEED_WORDS) != hipSuccess) {
+        ds->ctl = nullptr;
         rc = EPISDET_ERR_ALLOC;
+    }
+    if (rc == EPISDET_OK) {
+        unsigned char *at = (unsigned char *)(ds->ctl + 1);
+        ds->jobargs = at;
+        ds->jobstart = (unsigned long long *)(at + 1024);
+        ds->seed = (unsigned long long *)(at + 1024 + 256);
+    }
     for (int e = 0; e < 3 && rc == EPISDET_OK; e++)
         if (hipEventCreate(&ds->ev[e]) != hipSuccess) rc = EPISDET_ERR_HIP;
     if (rc == EPISDET_OK && hipHostMalloc((void **)&ds->stage, STAGE_BYTES, hipHostMallocMapped) != hipSuccess) {
@@ -1968,8 +1962,8 @@ void episdet_dataset_destroy(episdet_dataset *ds)
     if (ds->singles) (void)hipFree(ds->singles);
     if (ds->pairs) (void)hipFree(ds->pairs);
     if (ds->ctl) (void)hipFree(ds->ctl);
-    if (ds->jobargs) (void)hipFree(ds->jobargs);
-    if (ds->jobstart) (void)hipFree(ds->jobstart);
+    if (ds->gstart) (void)hipFree(ds->gstart);
+    if (ds->groups) (void)hipFree(ds->groups);
     if (ds->cand) (void)hipFree(ds->cand);
     if (ds->cand_s32) (void)hipFree(ds->cand_s32);
     if (ds->cand_s64) (void)hipFree(ds->cand_s64);
@@ -2108,6 +2102,8 @@ int episdet_run_noalloc(episdet_dataset *ds, const episdet_options *opt, episdet
         unsigned cand_cap;
         uint4 *pairs;
         ScoreTables tab;
+        unsigned long long *gstart;
+        int2 *groups;
         ~Bind()
         {
             t_scr = nullptr;
@@ -2120,9 +2116,12 @@ int episdet_run_noalloc(episdet_dataset *ds, const episdet_options *opt, episdet
             ds->cand_cap = cand_cap;
             ds->pairs = pairs;
             ds->tab[score] = tab;
+            ds->gstart = gstart;
+            ds->groups = groups;
         }
     } bind{ds,           opt->score,    ds->ctl,      ds->jobargs, ds->jobstart, ds->cand,
-           ds->cand_s32, ds->cand_s64, ds->cand_cap, ds->pairs,   ds->tab[opt->score]};
+           ds->cand_s32, ds->cand_s64, ds->cand_cap, ds->pairs,   ds->tab[opt->score],
+           ds->gstart,   ds->groups};
     ds->ctl = sp.ctl;
     ds->jobargs = sp.jobargs;
     ds->jobstart = sp.jobstart;
@@ -2130,6 +2129,8 @@ int episdet_run_noalloc(episdet_dataset *ds, const episdet_options *opt, episdet
     ds->cand_s32 = sp.cand_s32;
     ds->cand_s64 = sp.cand_s64;
     ds->cand_cap = SCRATCH_CAND;
+    ds->gstart = sp.gstart;
+    ds->groups = sp.groups;
     t_scr = &sp;
     return episdet_run(ds, opt, res);
 }
@@ -2243,7 +2244,7 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
             ds->n < o.order || o.topk > 1)
             return EPISDET_ERR_INVALID;
         const double tp = now_s();
-        if (o.rebuild) CHK(compute_singles(ds));
+        if (o.rebuild) CHK(compute_singles(ds, false));
         CHK(ensure_tables(ds, o.score));
         if (o.order == 3) CHK(ensure_pairs(ds, o.rebuild != 0));
         CHK(ensure_cand(ds, o.candidate_cap > 0 ? (unsigned)o.candidate_cap : DEFAULT_CAP));
@@ -2252,6 +2253,9 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         ktile[j] = o.tile;
         if (o.path == EPISDET_PATH_AUTO) CHK(choose_kernel(ds, o.order, o.score, &kpath[j], &ktile[j], o.autotune != 0));
     }
+    // the count tables are built on the datasets' streams, side by side; the
+    // graph runs on its own
+    for (int j = 0; j < njobs; j++) HIPCHK(hipStreamSynchronize(dss[j]->stream));
     // AUTO jobs of one order share one kernel: the MFMA tile their per-shape
     // choices give the most work (sets x samples).  One graph branch per order
     // packs the CUs better than one branch per tile: on the 64-job workload
@@ -2575,37 +2579,31 @@ static int dump_or_checksum(episdet_dataset *ds, int order, int path, int tile, 
     if (!tile_valid(order, mfma ? EPISDET_PATH_FUSED_MFMA : EPISDET_PATH_FUSED_VALU, tile)) return EPISDET_ERR_INVALID;
     const int nc = order == 3 ? 27 : 9;
     const unsigned long long total = episdet_n_choose_k((unsigned)ds->n, (unsigned)order);
+    if (total == 0) {                  // fewer SNPs than a set holds
+        if (checksum) *checksum = 0ull;
+        return EPISDET_OK;
+    }
     uint32_t *d_dump = nullptr;
     if (out) {
         if (capacity < total * 2 * nc) return EPISDET_ERR_INVALID;
         if (hipMalloc(&d_dump, sizeof(uint32_t) * total * 2 * nc) != hipSuccess) return EPISDET_ERR_ALLOC;
     }
     if (order == 3) CHK(ensure_pairs(ds));
-    CHK(init_ctl(ds));
     int rc;
-    unsigned long long *d_gstart = nullptr;
-    int2 *d_groups = nullptr;
     if (order == 3) {
-        std::vector<int2> groups;
-        std::vector<unsigned long long> gstart;
-        if (mfma) {
-            build_groups(ds->n, mfma_ty(tile), mfma_tz(tile), groups, gstart, mfma_xstep(tile));
-        } else {
-            const Tri3Tile t = TRI_TILES[tile];
-            build_groups(ds->n, 16 * t.A, 16 * t.B, groups, gstart);
-        }
-        if (hipMalloc(&d_gstart, sizeof(unsigned long long) * gstart.size()) != hipSuccess) return EPISDET_ERR_ALLOC;
-        if (hipMalloc(&d_groups, sizeof(int2) * std::max<size_t>(groups.size(), 1)) != hipSuccess) return EPISDET_ERR_ALLOC;
-        HIPCHK(hipMemcpy(d_gstart, gstart.data(), sizeof(unsigned long long) * gstart.size(), hipMemcpyHostToDevice));
-        if (!groups.empty())
-            HIPCHK(hipMemcpy(d_groups, groups.data(), sizeof(int2) * groups.size(), hipMemcpyHostToDevice));
+        const Tri3Tile vt = TRI_TILES[mfma ? 0 : tile];
+        const int t[3] = {mfma ? mfma_ty(tile) : 16 * vt.A, mfma ? mfma_tz(tile) : 16 * vt.B, mfma ? mfma_xstep(tile) : 1};
         TriArgs ta;
         fill_tri_common(ds, ta);
-        ta.gstart = d_gstart;
-        ta.groups = d_groups;
-        ta.ngroups = (int)groups.size();
-        ta.nunits = gstart.back();
+        rc = ensure_groups(ds, t, &ta.ngroups, &ta.nunits);
+        if (rc != EPISDET_OK) {
+            if (d_dump) (void)hipFree(d_dump);
+            return rc;
+        }
+        ta.gstart = ds->gstart;
+        ta.groups = ds->groups;
         ta.dump = d_dump;
+        CHK(init_single(ds, ta, ta.nunits));
         if (mfma)
             rc = out ? dispatch_tri_mfma<MODE_DUMP>(ds, tile, ta, ds->stream)
                      : dispatch_tri_mfma<MODE_CHECKSUM>(ds, tile, ta, ds->stream);
@@ -2616,12 +2614,11 @@ static int dump_or_checksum(episdet_dataset *ds, int order, int path, int tile, 
         PairArgs pa;
         fill_pairs(ds, pa, mfma, tile);
         pa.dump = d_dump;
+        CHK(init_single(ds, pa, pa.nunits));
         rc = out ? dispatch_pairs<MODE_DUMP>(ds, mfma, tile, pa, ds->stream)
                  : dispatch_pairs<MODE_CHECKSUM>(ds, mfma, tile, pa, ds->stream);
     }
     HIPCHK(hipStreamSynchronize(ds->stream));
-    if (d_gstart) (void)hipFree(d_gstart);
-    if (d_groups) (void)hipFree(d_groups);
     if (rc == EPISDET_OK && out)
         HIPCHK(hipMemcpy(out, d_dump, sizeof(uint32_t) * total * 2 * nc, hipMemcpyDeviceToHost));
     if (rc == EPISDET_OK && checksum) {
