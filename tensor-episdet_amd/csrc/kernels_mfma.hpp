@@ -368,6 +368,7 @@ __device__ __forceinline__ unsigned lds_addr(const void *p) { return (unsigned)(
 __device__ __forceinline__ void lds_dma16(i32x4_t rsrc, unsigned lds, unsigned voffset, unsigned soffset)
 {
     const unsigned m0 = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
+    soffset = (unsigned)__builtin_amdgcn_readfirstlane((int)soffset);   // uniform, wherever the compiler keeps it
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(m0), "v"(voffset), "s"(rsrc), "s"(soffset)

@@ -21,11 +21,17 @@
 //    loaded straight to LDS through the scalar buffer descriptor of its
 //    class, double-buffered: chunk t + 1 is issued after the barrier that
 //    starts chunk t;
-//  * after the last chunk the accumulators go to LDS in two halves (column
-//    tile 0, then 1, of every wave) and the 256 threads build and score
-//    eight pair tables per half.
-// LDS: 64 KB stage / dump area plus the ln m! table, so two workgroups fit a
-// CU and one's scoring runs beside the other's counting.
+//  * the B rows of a wave lie by plane, so its column tile cb is plane cb of 32
+//    B SNPs and a lane ends up with all eight counts of its 16 pairs (one B,
+//    16 A).  It bounds their scores in FP32 straight from its registers
+//    (quick_bound, about 85 vector instructions a pair); only the pairs that
+//    leaves go through LDS to integer tables and FP32 scores.  Before, every
+//    pair's counts went through LDS and both its classes' tables were derived
+//    first: pairs at 3001 x 9973 took 167 us a search, now 143, and 8192 x
+//    2000 0.67 ms of kernel time, now 0.25.
+// LDS: 64 KB stage / dump area, the ln m! table and the unit's single counts,
+// so two workgroups fit a CU and one's scoring runs beside the other's
+// counting.
 #pragma once
 #include "kernels_mfma_pairs.hpp"
 #include "kernels_mfma4.hpp"
@@ -41,7 +47,8 @@ constexpr int P3_LOADS = P3_ROWS / P3_ROWS_PER_LOAD;        // 32 per chunk
 constexpr int P3_LOADS_PER_WAVE = P3_LOADS / 4;             // 8
 constexpr int P3_BUF_WORDS = P3_ROWS * P3_KW;               // 8192 (32 KB)
 constexpr int P3_STAGE_WORDS = 2 * P3_BUF_WORDS;            // double-buffered (64 KB)
-constexpr int P3_DUMP_WORDS = 2 * 4 * 2 * 16 * 64;          // class x wave x row tile x reg x lane (64 KB)
+constexpr int P3_CLASS_WORDS = 2 * 8 * 64 * 2;              // a row tile's counts of a class: plane of B x A x lane x plane of A
+constexpr int P3_DUMP_WORDS = 4 * 2 * P3_CLASS_WORDS;       // wave x class (64 KB)
 constexpr int P3_SMEM_WORDS = P3_STAGE_WORDS > P3_DUMP_WORDS ? P3_STAGE_WORDS : P3_DUMP_WORDS;
 static_assert(P3_KW == M2_KW, "128-byte rows use the swizzle of m2_at");
 
@@ -55,7 +62,8 @@ __device__ __forceinline__ void p3_row_offsets(int W, int a0, int b0, int w, int
 #pragma unroll
     for (int k = 0; k < P3_LOADS_PER_WAVE; k++) {
         const int r = (w + 4 * k) * P3_ROWS_PER_LOAD + rl;
-        const int row = r < P3_AROWS ? 2 * a0 + r : 2 * b0 + (r - P3_AROWS);
+        const int rb = r - P3_AROWS;         // 64 (b / 32) + 32 plane + b % 32
+        const int row = r < P3_AROWS ? 2 * a0 + r : 2 * (b0 + (rb >> 6) * 32 + (rb & 31)) + ((rb >> 5) & 1);
         roff[k] = ((unsigned)row * (unsigned)W + (unsigned)(q * 4)) * 4u;
     }
 }
@@ -100,48 +108,106 @@ __device__ __forceinline__ void p3_chunk(const uint32_t *cur, int ar0, int ar1, 
     }
 }
 
+// A unit number with a pair in it, and its tiles: units of XCD blocks that lie
+// outside the triangle are passed over here, by the one thread that fetches,
+// while the others still contract.
+struct P3Unit {
+    unsigned long long uu;
+    int tA, tB;
+};
+__device__ __forceinline__ P3Unit p3_fetch(const BatchPair &bp)
+{
+    P3Unit r;
+    for (;;) {
+        r.uu = bp.xcd ? fetch_xcd(bp.queue, bp.total) : atomicAdd(bp.queue, 1ull);
+        if (r.uu >= bp.total) return r;
+        int j = 0;
+        while (j + 1 < bp.njobs && bp.job_start[j + 1] <= r.uu) j++;
+        const unsigned long long u = r.uu - bp.job_start[j];
+        if (!bp.jobs[j].blocked) {
+            unrank_tri(u, r.tA, r.tB);
+            return r;
+        }
+        if (blocked_unrank(u, bp.jobs[j].ntiles, r.tA, r.tB)) return r;
+    }
+}
+
+// Single counts of a unit's SNPs for quick_bound: T of genotypes 0, 1, 2 and
+// their D = cases - pi T, eight words each (two unused).
+__device__ __forceinline__ void p3_single(const PairArgs &p, int v, float *o)
+{
+    const Singles s = ld_global(p.singles, min(v, p.n - 1));
+    const uint32_t c2 = (uint32_t)p.N0 - s.x - s.y, t2 = (uint32_t)p.N1 - s.z - s.w;
+    const float T0 = (float)(s.x + s.z), T1 = (float)(s.y + s.w), T2 = (float)(c2 + t2), pi = p.sc.lb_pi;
+    *(float4 *)o = make_float4(T0, T1, T2, fmaf(-pi, T0, (float)s.x));
+    *(float4 *)(o + 4) = make_float4(fmaf(-pi, T1, (float)s.y), fmaf(-pi, T2, (float)c2), 0.f, 0.f);
+}
+
+// Quick bound of one pair from its counts c[class][plane of A][plane of B].
+__device__ __forceinline__ bool p3_quick(const ScoreCtx &sc, const float (&c)[2][2][2], const float4 &a0,
+                                         const float4 &a1, const float4 &b0, const float4 &b1, float thr, bool valid)
+{
+    float T[9], D[9];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            T[i * 3 + j] = c[0][i][j] + c[1][i][j];
+            D[i * 3 + j] = fmaf(-sc.lb_pi, T[i * 3 + j], c[0][i][j]);
+        }
+    auto derive = [](float (&t)[9], float A0, float A1, float A2, float B0, float B1) {
+        t[2] = (A0 - t[0]) - t[1];
+        t[5] = (A1 - t[3]) - t[4];
+        t[6] = (B0 - t[0]) - t[3];
+        t[7] = (B1 - t[1]) - t[4];
+        t[8] = (A2 - t[6]) - t[7];
+    };
+    derive(T, a0.x, a0.y, a0.z, b0.x, b0.y);
+    derive(D, a0.w, a1.x, a1.y, b0.w, b1.x);
+    return quick_bound<9>(sc, T, D, thr, valid);
+}
+
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void k_pairs_mfma2(BatchPair bp)
 {
     static_assert(MODE != MODE_PAIRTABLE, "the pair table is built by k_pairs_mfma");
     __shared__ __attribute__((aligned(16))) uint32_t smem[P3_SMEM_WORDS];
-    __shared__ unsigned long long s_u;
-    __shared__ float s_red[8];
+    __shared__ __attribute__((aligned(16))) float s_one[scores_sets(MODE) ? 128 * 8 : 4];    // 64 A, 64 B
+    __shared__ P3Unit s_u;
+    __shared__ unsigned s_best;
     __shared__ float s_lnf[scores_sets(MODE) ? LNF_SMALL : 1];
     if constexpr (scores_sets(MODE)) load_lnf(s_lnf);
     const int tid = threadIdx.x;
-    const int w = tid >> 6, lane = tid & 63, h = lane >> 5, i = lane & 31;
-    const int rp = w >> 1, cp = w & 1;
-    // LDS rows read by this lane: A rows of its two row tiles, B rows of its
-    // two column tiles (tile row / column i = 2 * snp + plane)
-    const int ar0 = 64 * rp + i, ar1 = 64 * rp + 32 + i;
-    const int br0 = P3_AROWS + 64 * cp + i, br1 = P3_AROWS + 64 * cp + 32 + i;
+    const int w = uniform(tid >> 6), rp = w >> 1, cp = w & 1;
 
-    int j = 0;
+    unsigned long long jfirst = 0, jend = 0;
+    PairArgs p;
+    if (tid == 0) s_u = p3_fetch(bp);
     for (;;) {
-        if (tid == 0) s_u = bp.xcd ? fetch_xcd(bp.queue, bp.total) : atomicAdd(bp.queue, 1ull);
         __syncthreads();
-        const unsigned long long uu = s_u;
+        const unsigned long long uu = uniform(s_u.uu);
         if (uu >= bp.total) break;
-        if (uu < bp.job_start[j]) j = 0;                  // per-XCD queues go out of order
-        while (j + 1 < bp.njobs && bp.job_start[j + 1] <= uu) j++;
-        const PairArgs &p = bp.jobs[j];
-        const unsigned long long u = uu - bp.job_start[j];
-        int tA, tB;
-        if (!p.blocked) {
-            unrank_tri(u, tA, tB);
-        } else if (!blocked_unrank(u, p.ntiles, tA, tB)) {
-            __syncthreads();       // every thread has read s_u before the next fetch writes it
-            continue;
+        const int a0 = uniform(s_u.tA) * P3_TA, b0 = uniform(s_u.tB) * P3_TB;
+        if (uu < jfirst || uu >= jend) {                  // per-XCD queues go out of order
+            int j = 0;
+            while (j + 1 < bp.njobs && ld_const(bp.job_start, (size_t)(j + 1)) <= uu) j++;
+            p = ld_const(bp.jobs, (size_t)j);
+            jfirst = ld_const(bp.job_start, (size_t)j);
+            jend = ld_const(bp.job_start, (size_t)(j + 1));
         }
-        const int a0 = tA * P3_TA, b0 = tB * P3_TB;
+        // LDS rows read by this lane: A rows of its two row tiles (tile row i =
+        // 2 snp + plane), B rows of its two planes (made per unit: they are not
+        // to hold registers through the scoring)
+        const int lane = opaque(tid & 63), h = lane >> 5, i = lane & 31;
+        const int ar0 = 64 * rp + i, ar1 = 64 * rp + 32 + i;
+        const int br0 = P3_AROWS + 64 * cp + i, br1 = P3_AROWS + 64 * cp + 32 + i;
         const int nch0 = p.W0 / P3_KW, nch = nch0 + p.W1 / P3_KW;
         const i32x4_t rs0 = m2_rsrc(p.p0, p.bytes0), rs1 = m2_rsrc(p.p1, p.bytes1);
         unsigned roff0[P3_LOADS_PER_WAVE], roff1[P3_LOADS_PER_WAVE];
         p3_row_offsets(p.W0, a0, b0, w, lane, roff0);
         p3_row_offsets(p.W1, a0, b0, w, lane, roff1);
 
-        v16f_t acc[2][2][2];                                // [class][row tile][column tile]
+        v16f_t acc[2][2][2];                                // [class][row tile][plane of B]
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
@@ -156,6 +222,12 @@ __global__ __launch_bounds__(256, 2) void k_pairs_mfma2(BatchPair bp)
             if (nch0 > 0) p3_issue_buf(rs0, roff0, 0, lds_addr(smem), w);
             else p3_issue_buf(rs1, roff1, 0, lds_addr(smem), w);
         }
+        if constexpr (scores_sets(MODE)) {
+            const int e = opaque(tid);
+            if (e < 128) p3_single(p, e < 64 ? a0 + e : b0 + e - 64, s_one + e * 8);
+        }
+        P3Unit next{};
+        unsigned best = 0;
         // two loops, one per class, so each contracts into one fixed set of
         // accumulators
 #pragma unroll
@@ -169,82 +241,143 @@ __global__ __launch_bounds__(256, 2) void k_pairs_mfma2(BatchPair bp)
                     uint32_t *nb = smem + (tn & 1) * P3_BUF_WORDS;
                     if (tn < nch0) p3_issue_buf(rs0, roff0, tn * P3_KW, lds_addr(nb), w);
                     else p3_issue_buf(rs1, roff1, (tn - nch0) * P3_KW, lds_addr(nb), w);
+                } else if (tid == 0) {
+                    // the next unit and the score bound arrive while the last
+                    // chunk is contracted
+                    next = p3_fetch(bp);
+                    if constexpr (scores_sets(MODE))
+                        best = __hip_atomic_load(p.co.best_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 p3_chunk(smem + (t & 1) * P3_BUF_WORDS, ar0, ar1, br0, br1, h, acc[c]);
             }
         }
         __builtin_amdgcn_s_waitcnt(0);
+        if (tid == 0) {
+            s_u = next;
+            s_best = best;
+        }
         __syncthreads();
 
-        float bad[16];
-        unsigned long long packed[16];
+        // Each wave scores what it counted.  Output register r = 4 q + 2 s + i
+        // of row tile rb holds, in lane 32 h + b, A = 16 rb + 4 q + 2 h + s,
+        // plane i, against B = b.
+        const int ln = opaque(tid & 63), eh = ln >> 5, eb = ln & 31;
+        const int A0 = a0 + 32 * rp + 2 * eh, B = b0 + 32 * cp + eb;
         unsigned long long hsum = 0;
         // sets whose badness lower bound is above this cannot become
         // candidates; their FP32 score is skipped (skip_threshold)
-        float skip_above = INFINITY;
-        if constexpr (scores_sets(MODE)) skip_above = skip_threshold(p.sc, p.co.best_key);
+        float thr = INFINITY;
+        if constexpr (scores_sets(MODE)) thr = skip_threshold(p.sc, s_best);
+        // counts of a row tile -> LDS [class][plane of B][m][lane][plane of A], m = 2 q + s;
+        // read by this wave alone
+        float *dump = (float *)smem + w * 2 * P3_CLASS_WORDS;
+        auto put = [&](const v16f_t &v, int cls, int cb) {
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-            // column tile hf of every wave -> LDS [class][wave][row tile][reg][lane]
+            for (int m = 0; m < 8; m++) {
+                const int r = 4 * (m >> 1) + 2 * (m & 1);
+                *(float2 *)&dump[cls * P3_CLASS_WORDS + ((cb * 8 + m) * 64 + ln) * 2] = make_float2(v[r], v[r + 1]);
+            }
+        };
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++) put(acc[c][0][cb], c, cb);
+        __builtin_amdgcn_wave_barrier();
+        const float4 *oneB = (const float4 *)(s_one + (64 + 32 * cp + eb) * 8);
+        // rolled, so the kernel holds the scoring code once
+#pragma unroll 1
+        for (int rb = 0;; rb++) {
+            const int A1 = A0 + 16 * rb;
+            auto read = [&](int m, float2 (&v)[2][2]) {     // [class][plane of B]
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        v[c][j] = *(const float2 *)&dump[c * P3_CLASS_WORDS + ((j * 8 + m) * 64 + ln) * 2];
+            };
+            // bit m: this lane's pair with A1 + 4 q + s is not ruled out
+            unsigned todo = 0;
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                const int A = A1 + 4 * (m >> 1) + (m & 1);
+                todo |= (A < B && B < p.n) ? 1u << m : 0u;
+            }
+            // While no bound is known (a search's first units: half of them at
+            // 3001 x 9973), one pair per lane is scored and the bound read again
+            // before the rest is bounded.
+            bool quick = scores_sets(MODE) && thr < INFINITY;
+#pragma unroll 1
+            for (;;) {
+                if constexpr (scores_sets(MODE)) {
+                    if (quick && p.sc.fb_scale > 0.f && __ballot(todo != 0)) {
+                        const float4 b0v = oneB[0], b1v = oneB[1];
+                        const float4 *oneA = (const float4 *)(s_one + (32 * rp + 16 * rb + 2 * eh) * 8);
+                        unsigned keep = 0;
+#pragma unroll 2
+                        for (int m = 0; m < 8; m++) {
+                            float2 v[2][2];
+                            read(m, v);
+                            const float4 *o = oneA + (4 * (m >> 1) + (m & 1)) * 2;
+                            const float c[2][2][2] = {{{v[0][0].x, v[0][1].x}, {v[0][0].y, v[0][1].y}},
+                                                      {{v[1][0].x, v[1][1].x}, {v[1][0].y, v[1][1].y}}};
+                            keep |= p3_quick(p.sc, c, o[0], o[1], b0v, b1v, thr, (todo >> m) & 1u) ? 0u : 1u << m;
+                        }
+                        todo &= keep;
+                    }
+                    quick = false;
+                }
+                if (!__ballot(todo != 0)) break;
+                float bad = INFINITY;
+                unsigned long long packed = 0;
+                if (todo) {
+                    const int m = __ffs(todo) - 1;
+                    todo &= todo - 1;
+                    const int A = A1 + 4 * (m >> 1) + (m & 1);
+                    float2 v[2][2];
+                    read(m, v);
+                    uint32_t n4[2][4];
+#pragma unroll
+                    for (int c = 0; c < 2; c++)
+#pragma unroll
+                        for (int j = 0; j < 2; j++) {
+                            n4[c][j] = (uint32_t)v[c][j].x;
+                            n4[c][2 + j] = (uint32_t)v[c][j].y;
+                        }
+                    const Singles sa = ld_global(p.singles, A), sb = ld_global(p.singles, B);
+                    uint32_t cas[9], ctl[9];
+                    pair9(n4[0][0], n4[0][1], n4[0][2], n4[0][3], sa.x, sa.y, sb.x, sb.y, (uint32_t)p.N0, cas);
+                    pair9(n4[1][0], n4[1][1], n4[1][2], n4[1][3], sa.z, sa.w, sb.z, sb.w, (uint32_t)p.N1, ctl);
+                    packed = (unsigned long long)A | ((unsigned long long)B << 32);
+                    if constexpr (scores_sets(MODE)) {
+                        if (!(thr < INFINITY && p.sc.fb_scale == 0.f && bound_exceeds<9>(p.sc, cas, ctl, thr)))
+                            bad = badness_f32_flat<9>(p.sc, cas, ctl, s_lnf);
+                    } else if constexpr (MODE == MODE_DUMP) {
+                        uint32_t *o = p.dump + rank2(A, B) * 18;
+                        for (int c = 0; c < 9; c++) {
+                            o[c] = cas[c];
+                            o[9 + c] = ctl[c];
+                        }
+                    } else if constexpr (MODE == MODE_CHECKSUM) {
+                        hsum += table_hash(rank2(A, B), cas, ctl, 9);
+                    }
+                }
+                if constexpr (MODE == MODE_SEARCH) publish_wave(p.co, p.sc.margin, bad, packed);
+                if constexpr (MODE == MODE_TOPK) publish_wave_topk(p.co, p.sc.margin, bad, packed);
+                if constexpr (scores_sets(MODE)) {
+                    if (!(thr < INFINITY)) {
+                        thr = skip_threshold(p.sc, __hip_atomic_load(p.co.best_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                        quick = thr < INFINITY;
+                    }
+                }
+            }
+            if (rb) break;
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int c = 0; c < 2; c++)
 #pragma unroll
-                for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        smem[((((c * 4 + w) * 2 + rb) * 16) + r) * 64 + lane] = (uint32_t)acc[c][rb][hf][r];
-            __syncthreads();
-#pragma unroll
-            for (int q8 = 0; q8 < 8; q8++) {
-                const int m = hf * 8 + q8;
-                const int T = q8 * 256 + tid;                   // 64 A x 32 B of this half
-                const int al = T >> 5, bsel = T & 31;
-                const int tcp = bsel >> 4, b16 = bsel & 15;
-                const int bl = 32 * tcp + 16 * hf + b16;
-                const int A = a0 + al, B = b0 + bl;
-                bad[m] = INFINITY;
-                packed[m] = (unsigned long long)A | ((unsigned long long)B << 32);
-                if (!(A < B && B < p.n)) continue;
-                // row 2*al + pi lives in the waves of row pair al/32, row tile
-                // (al/16)%2, tile row rho = 2*(al%16) + pi; column 2*bl + pj
-                // in the wave of column pair bl/32, column tile hf, tile
-                // column 2*(bl%16) + pj.  Output register r = 4*(rho/8) +
-                // rho%4 of lane 32*((rho/4)%2) + column.
-                const int tw = (al >> 5) * 2 + tcp, trb = (al >> 4) & 1, a16 = al & 15;
-                uint32_t n4c[4], n4t[4];
-#pragma unroll
-                for (int pi = 0; pi < 2; pi++)
-#pragma unroll
-                    for (int pj = 0; pj < 2; pj++) {
-                        const int rho = 2 * a16 + pi;
-                        const int reg = 4 * (rho >> 3) + (rho & 3);
-                        const int ln = 32 * ((rho >> 2) & 1) + 2 * b16 + pj;
-                        const int off = (((tw * 2 + trb) * 16) + reg) * 64 + ln;
-                        n4c[pi * 2 + pj] = smem[0 * 4 * 2 * 16 * 64 + off];
-                        n4t[pi * 2 + pj] = smem[1 * 4 * 2 * 16 * 64 + off];
-                    }
-                const Singles sa = ld_global(p.singles, A), sb = ld_global(p.singles, B);
-                uint32_t cas[9], ctl[9];
-                pair9(n4c[0], n4c[1], n4c[2], n4c[3], sa.x, sa.y, sb.x, sb.y, (uint32_t)p.N0, cas);
-                pair9(n4t[0], n4t[1], n4t[2], n4t[3], sa.z, sa.w, sb.z, sb.w, (uint32_t)p.N1, ctl);
-                if constexpr (scores_sets(MODE)) {
-                    if (skip_above < INFINITY && bound_exceeds<9>(p.sc, cas, ctl, skip_above))
-                        continue;                           // bad[m] stays INFINITY
-                    bad[m] = badness_f32(p.sc, cas, ctl, s_lnf);
-                } else if constexpr (MODE == MODE_DUMP) {
-                    uint32_t *o = p.dump + rank2(A, B) * 18;
-                    for (int c = 0; c < 9; c++) {
-                        o[c] = cas[c];
-                        o[9 + c] = ctl[c];
-                    }
-                } else if constexpr (MODE == MODE_CHECKSUM) {
-                    hsum += table_hash(rank2(A, B), cas, ctl, 9);
-                }
-            }
-            __syncthreads();
+                for (int cb = 0; cb < 2; cb++) put(acc[c][1][cb], c, cb);
+            __builtin_amdgcn_wave_barrier();
         }
-        if constexpr (MODE == MODE_SEARCH) publish_candidates<16, 4>(p.co, p.sc.margin, bad, packed, s_red);
-        if constexpr (MODE == MODE_TOPK) publish_topk<16, 4>(p.co, p.sc.margin, bad, packed);
         if constexpr (MODE == MODE_CHECKSUM) {
             if (hsum) atomicAdd(p.checksum, hsum);
         }

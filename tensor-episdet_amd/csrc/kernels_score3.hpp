@@ -304,10 +304,10 @@ __device__ __forceinline__ void s3_read(const float *cnt, int cls_stride, int q,
 // lane half) and Z (one per lane of a half), whose counts start at cnt (cases;
 // controls cls_stride words on).  xy: the unit's (X, Y) marginals from
 // (X, y) on; e: the lane's entry of its (X, Z) marginals; yz: the (Y, Z) counts
-// of q = 0; thr: skip_threshold.
+// of q = 0; thr: skip_threshold, read again while it is +inf.
 template <int MODE>
 __device__ __forceinline__ void s3_score(const TriArgs &p, const float *cnt, int cls_stride, const S3Pairs &s,
-                                         const float *xy, int e, S3Yz yz, int X, int y, int Z, int lane, float thr,
+                                         const float *xy, int e, S3Yz yz, int X, int y, int Z, int lane, float &thr,
                                          const float *s_lnf, unsigned long long &hsum)
 {
     const int h = lane >> 5;
@@ -317,48 +317,54 @@ __device__ __forceinline__ void s3_score(const TriArgs &p, const float *cnt, int
         const int Y = y + 2 * q + h;
         todo |= (X < Y && Y < Z && Z < p.n) ? 1u << q : 0u;
     }
-    if constexpr (scores_sets(MODE)) {
-        if (thr < INFINITY && p.sc.fb_scale > 0.f && __ballot(todo != 0)) {
-            S3Lane xz;
-            s3_lane(s, e, xz);
-            unsigned keep = 0;
+    // While no bound is known (the first units of a search that is not seeded),
+    // one triplet per lane is scored and the bound read again before the rest
+    // is bounded.
+    bool quick = scores_sets(MODE) && thr < INFINITY;
 #pragma unroll 1
-            for (int q = 0; q < 4; q++) {
-                const uint4 c0 = yz.c0, c1 = yz.c1;
-                if (q < 3) s3_yz(p, y + 2 * q + 2 + h, Z, yz);
-                float4 c[2][2];
-                s3_read(cnt, cls_stride, q, lane, c);
-                const float4 *xyq = (const float4 *)(xy + (2 * q + h) * 12);
-                const float4 e0 = xyq[0], e1 = xyq[1], e2 = xyq[2];
-                const float xyT[6] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y};
-                const float xyD[6] = {e2.x, e2.y, e2.z, e2.w, e1.z, e1.w};
-                const float pi = p.sc.lb_pi;
-                const float yzT[4] = {(float)(c0.x + c1.x), (float)(c0.y + c1.y), (float)(c0.z + c1.z),
-                                      (float)(c0.w + c1.w)};
-                const float yzD[4] = {fmaf(-pi, yzT[0], (float)c0.x), fmaf(-pi, yzT[1], (float)c0.y),
-                                      fmaf(-pi, yzT[2], (float)c0.z), fmaf(-pi, yzT[3], (float)c0.w)};
-                float T[27], D[27];
+    for (;;) {
+        if constexpr (scores_sets(MODE)) {
+            if (quick && p.sc.fb_scale > 0.f && __ballot(todo != 0)) {
+                S3Lane xz;
+                s3_lane(s, e, xz);
+                unsigned keep = 0;
+#pragma unroll 1
+                for (int q = 0; q < 4; q++) {
+                    const uint4 c0 = yz.c0, c1 = yz.c1;
+                    if (q < 3) s3_yz(p, y + 2 * q + 2 + h, Z, yz);
+                    float4 c[2][2];
+                    s3_read(cnt, cls_stride, q, lane, c);
+                    const float4 *xyq = (const float4 *)(xy + (2 * q + h) * 12);
+                    const float4 e0 = xyq[0], e1 = xyq[1], e2 = xyq[2];
+                    const float xyT[6] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y};
+                    const float xyD[6] = {e2.x, e2.y, e2.z, e2.w, e1.z, e1.w};
+                    const float pi = p.sc.lb_pi;
+                    const float yzT[4] = {(float)(c0.x + c1.x), (float)(c0.y + c1.y), (float)(c0.z + c1.z),
+                                          (float)(c0.w + c1.w)};
+                    const float yzD[4] = {fmaf(-pi, yzT[0], (float)c0.x), fmaf(-pi, yzT[1], (float)c0.y),
+                                          fmaf(-pi, yzT[2], (float)c0.z), fmaf(-pi, yzT[3], (float)c0.w)};
+                    float T[27], D[27];
 #pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const float a[4] = {c[0][k].x, c[0][k].y, c[0][k].z, c[0][k].w};
-                    const float b[4] = {c[1][k].x, c[1][k].y, c[1][k].z, c[1][k].w};
+                    for (int k = 0; k < 2; k++) {
+                        const float a[4] = {c[0][k].x, c[0][k].y, c[0][k].z, c[0][k].w};
+                        const float b[4] = {c[1][k].x, c[1][k].y, c[1][k].z, c[1][k].w};
 #pragma unroll
-                    for (int ij = 0; ij < 4; ij++) {
-                        const int cell = EPI_C3(ij >> 1, ij & 1, k);
-                        T[cell] = a[ij] + b[ij];
-                        D[cell] = fmaf(-pi, T[cell], a[ij]);
+                        for (int ij = 0; ij < 4; ij++) {
+                            const int cell = EPI_C3(ij >> 1, ij & 1, k);
+                            T[cell] = a[ij] + b[ij];
+                            D[cell] = fmaf(-pi, T[cell], a[ij]);
+                        }
                     }
+                    derive27(T, xyT, xz.T, yzT);
+                    derive27(D, xyD, xz.D, yzD);
+                    keep |= quick_bound<27>(p.sc, T, D, thr, (todo >> q) & 1u) ? 0u : 1u << q;
                 }
-                derive27(T, xyT, xz.T, yzT);
-                derive27(D, xyD, xz.D, yzD);
-                keep |= quick_bound<27>(p.sc, T, D, thr, (todo >> q) & 1u) ? 0u : 1u << q;
+                todo &= keep;
             }
-            todo &= keep;
+            quick = false;
         }
-    }
-    // what is left, one triplet per lane and turn
-#pragma unroll 1
-    while (__ballot(todo != 0)) {
+        // what is left, one triplet per lane and turn
+        if (!__ballot(todo != 0)) break;
         float bad = INFINITY;
         unsigned long long packed = 0;
         if (todo) {
@@ -395,6 +401,14 @@ __device__ __forceinline__ void s3_score(const TriArgs &p, const float *cnt, int
         }
         if constexpr (MODE == MODE_SEARCH) publish_wave(p.co, p.sc.margin, bad, packed);
         if constexpr (MODE == MODE_TOPK) publish_wave_topk(p.co, p.sc.margin, bad, packed);
+        if constexpr (scores_sets(MODE)) {
+            if (!(thr < INFINITY)) {
+                thr = skip_threshold(p.sc, __hip_atomic_load(p.co.best_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                quick = thr < INFINITY;
+            }
+            if (quick) s3_yz(p, y + h, Z, yz);
+            else yz = S3Yz{};               // not held through the scoring above
+        }
     }
 }
 

@@ -1124,9 +1124,9 @@ int issue_fused(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned long long
     if (order == 3) CHK(init_single(ds, ta, ta.nunits, u0, seed_key));
     else CHK(init_single(ds, pa, pa.nunits, u0, seed_key));
     if (pl.seed_pairs > 0) CHK(seed_from_pairs(ds, pl, topk));
-    // the 3-way kernels that tighten the top-k bound from the candidates' own
-    // scores (tighten_topk) must find +inf in slots not written yet
-    if (topk && order == 3 && mfma && tile >= 3) {
+    // the kernels that tighten the top-k bound from the candidates' own scores
+    // (tighten_topk) must find +inf in slots not written yet
+    if (topk && mfma && (order == 3 ? tile >= 3 : tile == 1)) {
         hipLaunchKernelGGL(k_fill_f32, dim3(4 * ds->cu), dim3(256), 0, ds->stream, ds->cand_s32, cap, INFINITY);
         HIPCHK(hipGetLastError());
     }

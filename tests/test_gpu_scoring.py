@@ -1,7 +1,7 @@
-"""Scoring of the 3-way kernels' work units (MFMA tiles 3, 4 and 5): the sets
-at the edges of a unit (X pairs, 32 Y, 32 Z), classes of one and several
-chunks, and the top-k bound that the kernels tighten from their own candidates.
-Winners, rankings and FP64 scores are the oracle's, bit for bit."""
+"""Scoring of the MFMA kernels' work units: the sets at the edges of a 3-way
+unit (tiles 3, 4 and 5: X pairs, 32 Y, 32 Z) and of a 2-way one, classes of one
+and several chunks, and the top-k bound that the kernels tighten from their own
+candidates.  Winners, rankings and FP64 scores are the oracle's, bit for bit."""
 import math
 
 import pytest
@@ -28,3 +28,21 @@ def test_unit_edges(n, Nc, Nt, score):
                 p, s, _ = ds.topk(3, k, score=score, path=episdet.PATH_FUSED_MFMA, tile=tile)
                 m = min(k, math.comb(n, 3))
                 assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
+
+
+@pytest.mark.parametrize("n,Nc,Nt", [(2, 1, 1), (63, 40, 25), (64, 1024, 1025), (65, 3000, 31), (130, 700, 2049),
+                                     (1030, 600, 500)])
+@pytest.mark.parametrize("score", [episdet.K2, episdet.MI])
+def test_pair_unit_edges(n, Nc, Nt, score):
+    """The 2-way kernel's 64 x 64 units (MFMA tile 1), in triangular order and
+    (from 16 tiles up) in XCD blocks."""
+    syn = episdet.generate(n, Nc, Nt, seed=400 + n, planted_sets=1 if n >= 64 else 0, planted_order=2)
+    ref_p, ref_s = O.ranked(syn.cases, syn.controls, Nc, Nt, 2, score)
+    with episdet.Dataset.from_synthetic(syn) as ds:
+        print(f"pair edges n={n} Nc={Nc} Nt={Nt} score={score}", flush=True)
+        r = ds.run(2, score, path=episdet.PATH_FUSED_MFMA, tile=1)
+        assert r["packed"] == int(ref_p[0]) and r["best_score"] == float(ref_s[0])
+        for k in (2, 65, 1024):
+            p, s, _ = ds.topk(2, k, score=score, path=episdet.PATH_FUSED_MFMA, tile=1)
+            m = min(k, math.comb(n, 2))
+            assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
