@@ -119,7 +119,15 @@ __device__ float g_lnfact[LNF_SMALL];
 
 __device__ __forceinline__ void load_lnf(float *s_lnf)
 {
-    for (int i = threadIdx.x; i < LNF_SMALL; i += blockDim.x) s_lnf[i] = g_lnfact[i];
+    // four loads in flight per turn (one turn for 256 threads)
+    for (int i = threadIdx.x; i < LNF_SMALL; i += 4 * blockDim.x) {
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = i + k * (int)blockDim.x < LNF_SMALL ? g_lnfact[i + k * blockDim.x] : 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i + k * (int)blockDim.x < LNF_SMALL) s_lnf[i + k * blockDim.x] = v[k];
+    }
 }
 
 // K2 term T'(m) = ln m! - c*m, c = ln N - 1.
@@ -244,6 +252,50 @@ __device__ __forceinline__ float mi_f32(const uint32_t *cas, const uint32_t *ctl
     return s * scale;
 }
 
+// mi_f32 as k2_f32_flat is k2_f32: three cells a turn, both forms of mi_dterm
+// computed and one chosen; the same FP32 MI.
+template <int NC>
+__device__ __forceinline__ float mi_f32_flat(const uint32_t *cas, const uint32_t *ctl, const float (&q)[2], float scale)
+{
+#pragma clang fp contract(off)
+    static_assert(NC % 3 == 0, "whole turns");
+    auto term = [](uint32_t x, uint32_t n, float qc) {
+        const float nf = (float)n, y = qc * nf;
+        const float d = fmaf(-qc, nf, (float)x);
+        const float e = d * __builtin_amdgcn_rcpf(y);
+        const float t = -e;
+        float s = 1.f / 132.f;
+        s = fmaf(s, t, 1.f / 110.f);
+        s = fmaf(s, t, 1.f / 90.f);
+        s = fmaf(s, t, 1.f / 72.f);
+        s = fmaf(s, t, 1.f / 56.f);
+        s = fmaf(s, t, 1.f / 42.f);
+        s = fmaf(s, t, 1.f / 30.f);
+        s = fmaf(s, t, 1.f / 20.f);
+        s = fmaf(s, t, 1.f / 12.f);
+        s = fmaf(s, t, 1.f / 6.f);
+        s = fmaf(s, t, 0.5f);
+        const float near = (d * e) * s;
+        const float r = 1.f + e, lr = __builtin_amdgcn_logf(r) * LN2_F;
+        const float far = y * fmaf(r, lr, 1.f - r);
+        const float v = fabsf(e) <= 0.25f ? near : far;
+        return n == 0u ? 0.f : (x == 0u ? y : v);
+    };
+    float s = 0.f;
+#pragma unroll 1
+    for (int i = 0; i < NC; i += 3) {
+        float f[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const uint32_t n = cas[i + k] + ctl[i + k];
+            f[k] = term(cas[i + k], n, q[0]) + term(ctl[i + k], n, q[1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) s += f[k];
+    }
+    return s * scale;
+}
+
 // Lower bound of a table's badness (K2, or -MI), from
 //   KL(p || pi) <= K (p - pi)^2 on [0, 1],  K = max(-ln(1-pi)/pi^2, -ln(pi)/(1-pi)^2)
 // (the largest KL(p||pi)/(p-pi)^2, reached at p = 0 or 1) and the chi-square
@@ -313,7 +365,7 @@ __device__ __forceinline__ float badness_f32_flat(const ScoreCtx &sc, const uint
                                                   const float *s_lnf)
 {
     if (sc.score == SCORE_K2) return k2_f32_flat<NC>(cas, ctl, sc.invN, sc.k0, sc.c, sc.k2_total, s_lnf);
-    return -mi_f32(cas, ctl, NC, sc.mi_q, sc.mi_scale);
+    return -mi_f32_flat<NC>(cas, ctl, sc.mi_q, sc.mi_scale);
 }
 
 // ---------------------------------------------------------------- FP64 --

@@ -287,9 +287,9 @@ __device__ __forceinline__ void pair_count_class(const uint32_t *__restrict__ ba
 
 __host__ __device__ inline void unrank_tri(unsigned long long u, int &ta, int &tb)
 {
-    // u = tb*(tb+1)/2 + ta, 0 <= ta <= tb
-    double d = sqrt(8.0 * (double)u + 1.0);
-    long long b = (long long)((d - 1.0) * 0.5);
+    // u = tb*(tb+1)/2 + ta, 0 <= ta <= tb; FP32 puts tb within a few of its
+    // value (FP64 roots cost a fetching thread ten times the cycles)
+    long long b = (long long)((sqrtf(8.f * (float)u + 1.f) - 1.f) * 0.5f);
     while ((unsigned long long)(b + 1) * (unsigned long long)(b + 2) / 2 <= u) b++;
     while ((unsigned long long)b * (unsigned long long)(b + 1) / 2 > u) b--;
     tb = (int)b;
@@ -371,6 +371,35 @@ struct BatchPair {
     int xcd = 0;
 };
 
+// Uniform reads.  A unit number comes out of LDS and its job's argument block
+// and group out of global memory, so to the compiler every field is a vector
+// load, made again after each store or barrier, and every use waits for one.
+// The unit number is made uniform (readfirstlane) and the blocks, which no
+// kernel writes, are read through the constant address space: scalar loads,
+// once per unit, into scalar registers.  A 3-way MI search of 1000 SNPs x
+// 4000 samples went from 7.30 to 6.65 ms with that alone.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ unsigned long long uniform(unsigned long long v)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+template <typename T>
+__device__ __forceinline__ T ld_const(const T *p, size_t i)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    typedef const __attribute__((address_space(4))) unsigned *cptr_t;
+    const cptr_t src = (cptr_t)(p + i);
+    union {
+        T v;
+        unsigned w[sizeof(T) / 4];
+    } u;
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(T) / 4; k++) u.w[k] = src[k];
+    return u.v;
+}
+
 template <int R, int MODE>
 __global__ __launch_bounds__(256) void k_pairs_valu(BatchPair bp)
 {
@@ -386,11 +415,11 @@ __global__ __launch_bounds__(256) void k_pairs_valu(BatchPair bp)
     for (;;) {
         if (tid == 0) s_u = atomicAdd(bp.queue, 1ull);
         __syncthreads();
-        const unsigned long long uu = s_u;
+        const unsigned long long uu = uniform(s_u);
         if (uu >= bp.total) break;
-        while (j + 1 < bp.njobs && bp.job_start[j + 1] <= uu) j++;
-        const PairArgs &p = bp.jobs[j];
-        const unsigned long long u = uu - bp.job_start[j];
+        while (j + 1 < bp.njobs && ld_const(bp.job_start, (size_t)(j + 1)) <= uu) j++;
+        const PairArgs p = ld_const(bp.jobs, (size_t)j);
+        const unsigned long long u = uu - ld_const(bp.job_start, (size_t)j);
         int tA, tB;
         unrank_tri(u, tA, tB);
         const int a0 = tA * T, b0 = tB * T;
@@ -427,7 +456,7 @@ __global__ __launch_bounds__(256) void k_pairs_valu(BatchPair bp)
                     if constexpr (scores_sets(MODE)) {
                         if (skip_above < INFINITY && bound_exceeds<9>(p.sc, cas, ctl, skip_above))
                             continue;                           // bad[m] stays INFINITY
-                        bad[m] = badness_f32(p.sc, cas, ctl, s_lnf);
+                        bad[m] = badness_f32_flat<9>(p.sc, cas, ctl, s_lnf);
                     } else if constexpr (MODE == MODE_DUMP) {
                         uint32_t *o = p.dump + rank2(A, B) * 18;
                         for (int c = 0; c < 9; c++) {
@@ -469,35 +498,6 @@ struct TriArgs {
     int X, yb, zb;
     uint32_t *counts;                    // [2][256][256][8]
 };
-
-// Uniform reads.  A unit number comes out of LDS and its job's argument block
-// and group out of global memory, so to the compiler every field is a vector
-// load, made again after each store or barrier, and every use waits for one.
-// The unit number is made uniform (readfirstlane) and the blocks, which no
-// kernel writes, are read through the constant address space: scalar loads,
-// once per unit, into scalar registers.  A 3-way MI search of 1000 SNPs x
-// 4000 samples went from 7.30 to 6.65 ms with that alone.
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ unsigned long long uniform(unsigned long long v)
-{
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
-    return ((unsigned long long)hi << 32) | lo;
-}
-template <typename T>
-__device__ __forceinline__ T ld_const(const T *p, size_t i)
-{
-    static_assert(sizeof(T) % 4 == 0, "whole words");
-    typedef const __attribute__((address_space(4))) unsigned *cptr_t;
-    const cptr_t src = (cptr_t)(p + i);
-    union {
-        T v;
-        unsigned w[sizeof(T) / 4];
-    } u;
-#pragma unroll
-    for (unsigned k = 0; k < sizeof(T) / 4; k++) u.w[k] = src[k];
-    return u.v;
-}
 
 // Group of unit u (uniform) when the workgroup's previous unit was in group
 // g0: a workgroup's units only increase.  A binary search over what is left;

@@ -1406,14 +1406,17 @@ int choose_kernel(episdet_dataset *ds, int order, int score, int *path, int *til
         g_tune[key] = TuneChoice{*path, *tile};
         return EPISDET_OK;
     }
-    // A small 2-way search on its own (not in a batch, whose graph runs MFMA
-    // kernels): the VALU kernel of 32 x 32 units spreads it over more
-    // workgroups than the MFMA kernel's 64 x 64 units, which leave most CUs
-    // idle.  Whole searches at N = 2048 through the Python API took 0.065 /
-    // 0.067 / 0.081 ms against 0.083 / 0.085 / 0.086 ms at 256 / 512 / 1024
-    // SNPs, and 0.138 against 0.109 ms at 512 SNPs x 16384 samples, so the
-    // VALU kernel is chosen below 1e9 set-samples.
+    // A small 2-way search of few samples on its own (not in a batch, whose
+    // graph runs MFMA kernels): the VALU kernel of 32 x 32 units spreads it
+    // over more workgroups than the MFMA kernel's 64 x 64 units, which leave
+    // most CUs idle.  Whole K2 searches at 2048 samples took 53 / 59 / 61 us
+    // against 73 / 76 / 69 us at 64 / 256 / 512 SNPs, but 77 against 73 us at 1024
+    // SNPs, and with more samples a unit's count is the longer part and the
+    // matrix cores win: 87 against 81 us at 256 x 8192, 155 against 98 us at 300 x
+    // 20000, 416 against 226 us at 100 x 100000.  So the VALU kernel is chosen
+    // below 1e9 set-samples and up to 4096 samples.
     if (single && order == 2 &&
+        ds->N[0] + ds->N[1] <= 4096 &&
         (double)episdet_n_choose_k((unsigned)ds->n, 2) * (double)(ds->N[0] + ds->N[1]) < 1e9) {
         *path = EPISDET_PATH_FUSED_VALU;
         *tile = 1;
