@@ -24,24 +24,26 @@ constexpr bool scores_sets(int mode) { return mode == MODE_SEARCH || mode == MOD
 
 // ------------------------------------------------------------ data prep --
 
-// Copies caller planes (rows of Win words) into the device layout (rows of
-// Wd words), clearing every bit at or past sample N and every SNP >= n.
-// dst holds nsnp_rows SNPs x 2 planes x Wd words; src holds n x 2 x Win.
+// Copies caller planes (rows of Win words) of SNPs snp0 .. snp0 + snps - 1 into
+// the device layout (rows of Wd words), clearing every bit at or past sample N
+// and every SNP >= n.  dst is the layout's start, src the rows from snp0 on
+// (device memory, or mapped host memory: the copy over the link is then this
+// kernel's reads).
 __global__ void k_repack(const uint32_t *__restrict__ src, int Win, uint32_t *__restrict__ dst, int Wd, int n,
-                         int nsnp_rows, int N)
+                         int snp0, int snps, int N)
 {
-    const size_t total = (size_t)nsnp_rows * 2 * Wd;
+    const size_t total = (size_t)snps * 2 * Wd, row0 = (size_t)snp0 * 2;
     const int Wv = (N + 31) / 32;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         size_t row = i / Wd;
         int w = (int)(i % Wd);
         uint32_t v = 0;
-        if ((int)(row >> 1) < n && w < Wv && w < Win) {
+        if ((int)((row0 + row) >> 1) < n && w < Wv && w < Win) {
             v = src[row * Win + w];
             int valid = N - w * 32;
             if (valid < 32) v &= 0xFFFFFFFFu << (32 - valid);
         }
-        dst[i] = v;
+        dst[row0 * Wd + i] = v;
     }
 }
 

@@ -17,6 +17,8 @@
 #include <cstdlib>
 #include <cstddef>
 #include <cstring>
+#include <atomic>
+#include <thread>
 #include <vector>
 #include <tuple>
 #include <mutex>
@@ -214,20 +216,106 @@ int check_device(int *cu)
     return EPISDET_OK;
 }
 
+// Runs f(part, parts) on up to `most` threads, in the calling one if no
+// other can be started.
+template <typename F>
+void on_threads(int most, F &&f)
+{
+    const int parts = std::max(1, std::min(most, (int)std::thread::hardware_concurrency()));
+    std::vector<std::thread> th;
+    int started = 1;
+    try {
+        th.reserve((size_t)parts);
+        for (; started < parts; started++) th.emplace_back(f, started, parts);
+    } catch (...) {
+        // the parts that got no thread run below
+    }
+    f(0, parts);
+    for (int p = started; p < parts; p++) f(p, parts);
+    for (std::thread &t : th) t.join();
+}
+
+// Pinned, device-mapped staging for dataset uploads, shared by the process: one
+// upload uses it at a time (another that finds it taken copies from pageable
+// memory), 24 MB at most, given back when the process exits.  The runtime
+// moves pageable memory at about 20 GB/s; six threads fill this and the repacking
+// kernel reads it over the link, 64 MB in about 1.6 ms.
+constexpr int UP_THREADS = 6;
+constexpr size_t UP_SLOT = 4u << 20;
+std::mutex g_up_mu;
+unsigned char *g_up = nullptr, *g_up_dev = nullptr;
+
+// Called with g_up_mu held.
+bool upload_pool()
+{
+    if (g_up) return true;
+    if (hipHostMalloc((void **)&g_up, UP_SLOT * UP_THREADS, hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) {
+        g_up = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipHostGetDevicePointer((void **)&g_up_dev, g_up, 0) != hipSuccess) {
+        (void)hipHostFree(g_up);
+        g_up = nullptr;
+        return false;
+    }
+    std::atexit([] { (void)hipHostFree(g_up); });
+    return true;
+}
+
+// One class's planes through the pool: each thread fills its slot with the
+// next SNPs' rows and launches their repacking, and waits for that before it fills the
+// slot again.  Called with g_up_mu held and the pool there.
+int upload_pooled(episdet_dataset *ds, int c, const unsigned *src, int in_w)
+{
+    const size_t snp_bytes = sizeof(uint32_t) * 2 * (size_t)in_w;
+    const int per = (int)std::max<size_t>(1, UP_SLOT / snp_bytes);
+    const int chunks = (ds->n + per - 1) / per;
+    std::atomic<int> next{0}, rc{EPISDET_OK};
+    const auto work = [&](int part, int) {
+        hipEvent_t ev = nullptr;
+        bool used = false;
+        if (hipSetDevice(ds->dev) != hipSuccess || hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            rc = EPISDET_ERR_HIP;
+            return;
+        }
+        for (int k = next++; k < chunks && rc == EPISDET_OK; k = next++) {
+            const int s0 = k * per, s1 = std::min(ds->n, s0 + per);
+            if (used && hipEventSynchronize(ev) != hipSuccess) rc = EPISDET_ERR_HIP;
+            std::memcpy(g_up + UP_SLOT * part, src + (size_t)s0 * 2 * in_w, snp_bytes * (size_t)(s1 - s0));
+            // the last chunk also clears the rows past the last SNP
+            const int snps = (k + 1 == chunks ? ds->nrows : s1) - s0;
+            const size_t words = (size_t)snps * 2 * ds->W[c];
+            hipLaunchKernelGGL(k_repack, dim3((unsigned)std::min<size_t>((words + 255) / 256, 4096)), dim3(256), 0,
+                               ds->stream, (const uint32_t *)(g_up_dev + UP_SLOT * part), in_w, ds->planes[c],
+                               ds->W[c], ds->n, s0, snps, ds->N[c]);
+            if (hipGetLastError() != hipSuccess || hipEventRecord(ev, ds->stream) != hipSuccess) rc = EPISDET_ERR_HIP;
+            used = true;
+        }
+        // the slot is not to be filled by the next upload while it is read
+        if (used && hipEventSynchronize(ev) != hipSuccess) rc = EPISDET_ERR_HIP;
+        (void)hipEventDestroy(ev);
+    };
+    on_threads(std::min(UP_THREADS, chunks), work);
+    return rc;
+}
+
 int ensure_cand(episdet_dataset *ds, unsigned cap)
 {
     if (ds->cand_cap >= cap) return EPISDET_OK;
     if (t_scr) return EPISDET_ERR_SCRATCH;           // the slots of `scratch` are all there is
     if (ds->cand) (void)hipFree(ds->cand);
-    if (ds->cand_s32) (void)hipFree(ds->cand_s32);
-    if (ds->cand_s64) (void)hipFree(ds->cand_s64);
     ds->cand = nullptr;
     ds->cand_s32 = nullptr;
     ds->cand_s64 = nullptr;
     ds->cand_cap = 0;
-    if (dev_malloc((void **)&ds->cand, sizeof(unsigned long long) * cap) != hipSuccess) return EPISDET_ERR_ALLOC;
-    if (dev_malloc((void **)&ds->cand_s32, sizeof(float) * cap) != hipSuccess) return EPISDET_ERR_ALLOC;
-    if (dev_malloc((void **)&ds->cand_s64, sizeof(double) * cap) != hipSuccess) return EPISDET_ERR_ALLOC;
+    // packed indices, FP64 scores and FP32 scores in one block
+    if (dev_malloc((void **)&ds->cand, (2 * sizeof(unsigned long long) + sizeof(float)) * (size_t)cap) != hipSuccess) {
+        ds->cand = nullptr;
+        return EPISDET_ERR_ALLOC;
+    }
+    ds->cand_s64 = (double *)(ds->cand + cap);
+    ds->cand_s32 = (float *)(ds->cand_s64 + cap);
     ds->cand_cap = cap;
     return EPISDET_OK;
 }
@@ -269,15 +357,21 @@ int ensure_tables(episdet_dataset *ds, int score)
     t.invN = (float)(1.0 / (double)N);
     t.k0 = (float)(0.5 * std::log((double)N) - 1.0 + 0.5 * std::log(2.0 * M_PI));
     if (score == EPISDET_SCORE_K2) {
+        // (lgamma_r: lgamma's own sign variable is shared by the threads)
+        on_threads(len >= (1 << 14) ? 8 : 1, [&](int part, int parts) {
+            const int m1 = (int)((long long)len * (part + 1) / parts);
+            int sign;
+            for (int m = (int)((long long)len * part / parts); m < m1; m++) h64[m] = lgamma_r((double)m + 1.0, &sign);
+        });
         double mx = 0;
-        for (int m = 0; m < len; m++) {
-            h64[m] = std::lgamma((double)m + 1.0);
-            mx = std::max(mx, std::fabs(h64[m] - t.shift_c * (double)m));
-        }
+        for (int m = 0; m < len; m++) mx = std::max(mx, std::fabs(h64[m] - t.shift_c * (double)m));
         t.t_max = mx;
     } else {
         h64[0] = 0.0;
-        for (int m = 1; m <= N; m++) h64[m] = std::log2((double)m / (double)N);
+        on_threads(len >= (1 << 14) ? 8 : 1, [&](int part, int parts) {
+            const int m1 = (int)((long long)N * (part + 1) / parts);
+            for (int m = 1 + (int)((long long)N * part / parts); m <= m1; m++) h64[m] = std::log2((double)m / (double)N);
+        });
     }
     // inside a no-allocation call the table and the error word live in
     // `scratch` (the caller restores the dataset's tables afterwards)
@@ -1927,10 +2021,22 @@ int episdet_dataset_create(const unsigned *cases, const unsigned *controls, int 
         ds->W[c] = ((Wv + W_ALIGN - 1) / W_ALIGN) * W_ALIGN;
         const size_t in_bytes = sizeof(uint32_t) * (size_t)numSNPs * 2 * in_w[c];
         const size_t dev_words = (size_t)ds->nrows * 2 * ds->W[c];
+        if (hipMalloc(&ds->planes[c], sizeof(uint32_t) * dev_words) != hipSuccess) {
+            rc = EPISDET_ERR_ALLOC;
+            break;
+        }
+        // Large planes go through the pinned pool (a pair search of 4096 x
+        // 65536 from host buffers: 5.4 ms without, 3.9 with); below 4 MB a class
+        // starting threads is the longer part, and a slot has to hold a SNP's rows.
+        if (in_bytes >= UP_SLOT && sizeof(uint32_t) * 2 * (size_t)in_w[c] <= UP_SLOT) {
+            std::unique_lock<std::mutex> lk(g_up_mu, std::try_to_lock);
+            if (lk.owns_lock() && upload_pool()) {
+                rc = upload_pooled(ds, c, src[c], in_w[c]);
+                continue;
+            }
+        }
         uint32_t *stage = nullptr;
-        if (hipMalloc(&ds->planes[c], sizeof(uint32_t) * dev_words) != hipSuccess ||
-            hipMalloc(&stage, in_bytes) != hipSuccess) {
-            if (stage) (void)hipFree(stage);
+        if (hipMalloc(&stage, in_bytes) != hipSuccess) {
             rc = EPISDET_ERR_ALLOC;
             break;
         }
@@ -1938,7 +2044,7 @@ int episdet_dataset_create(const unsigned *cases, const unsigned *controls, int 
         if (rc == EPISDET_OK) {
             const int grid = (int)std::min<size_t>((dev_words + 255) / 256, 65536);
             hipLaunchKernelGGL(k_repack, dim3(grid), dim3(256), 0, ds->stream, stage, in_w[c], ds->planes[c], ds->W[c],
-                               numSNPs, ds->nrows, ds->N[c]);
+                               numSNPs, 0, ds->nrows, ds->N[c]);
             if (hipGetLastError() != hipSuccess) rc = EPISDET_ERR_HIP;
         }
         if (hipStreamSynchronize(ds->stream) != hipSuccess) rc = EPISDET_ERR_HIP;
@@ -1968,8 +2074,6 @@ void episdet_dataset_destroy(episdet_dataset *ds)
     if (ds->gstart) (void)hipFree(ds->gstart);
     if (ds->groups) (void)hipFree(ds->groups);
     if (ds->cand) (void)hipFree(ds->cand);
-    if (ds->cand_s32) (void)hipFree(ds->cand_s32);
-    if (ds->cand_s64) (void)hipFree(ds->cand_s64);
     for (hipEvent_t e : ds->ev)
         if (e) (void)hipEventDestroy(e);
     if (ds->stage) (void)hipHostFree(ds->stage);

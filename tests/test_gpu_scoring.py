@@ -46,3 +46,20 @@ def test_pair_unit_edges(n, Nc, Nt, score):
             p, s, _ = ds.topk(2, k, score=score, path=episdet.PATH_FUSED_MFMA, tile=1)
             m = min(k, math.comb(n, 2))
             assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
+
+
+def test_upload_through_the_pinned_pool():
+    """Planes of 4 MB and more a class go to the device in chunks of whole SNPs
+    (239 of them here); the rows on both sides of a chunk's edge, the caller's
+    own padding and the last rows arrive whole."""
+    n, Nc, Nt, words = 300, 70001, 69000, 2190
+    syn = episdet.generate(n, Nc, Nt, seed=77, cases_words=words, controls_words=words, planted_sets=1,
+                           planted_order=2)
+    sets = [(0, 238), (238, 239), (239, 240), (1, 299), (237, 298)]
+    with episdet.Dataset.from_synthetic(syn) as ds:
+        t = ds.tables(2, sets)
+        for i, s in enumerate(sets):
+            assert (t[i, 0] == O.table_bits(syn.cases, Nc, s)).all() and (t[i, 1] == O.table_bits(syn.controls, Nt, s)).all()
+        for score in (episdet.K2, episdet.MI):
+            r, o = ds.run(2, score), O.search(syn.cases, syn.controls, Nc, Nt, 2, score)
+            assert r["packed"] == o["packed"] and r["best_score"] == o["score"]
