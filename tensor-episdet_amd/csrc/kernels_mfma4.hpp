@@ -18,8 +18,8 @@
 //    half as many barriers and load rounds per sample;
 //  * after the last chunk the accumulators go to LDS in two halves of 16 Y and
 //    each wave scores one X against 8 Y x 32 Z per half (s3_score).
-// LDS: at most 68 KB for the stage / dump area plus the ln m! table, so two
-// workgroups fit a CU.
+// LDS: at most 68 KB for the stage / dump area, the ln m! table and the unit's
+// pair marginals, 79.5 KB, so two workgroups fit a CU.
 #pragma once
 #include "kernels_mfma3.hpp"
 #include "kernels_score3.hpp"

@@ -20,8 +20,8 @@
 // Each A operand feeds two MFMAs instead of version 4's four, so the operand
 // work per MFMA is higher; AUTO picks this version when the classes differ
 // in size (see choose_kernel).
-// LDS: 64 KB for the stage (3 buffers of 17 KB) / dump area plus the ln m!
-// table, so two workgroups fit a CU.
+// LDS: 64 KB for the stage (3 buffers of 17 KB) / dump area, the ln m! table
+// and the unit's pair marginals, 75.5 KB, so two workgroups fit a CU.
 #pragma once
 #include "kernels_mfma4.hpp"
 

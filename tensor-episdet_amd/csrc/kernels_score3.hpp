@@ -5,10 +5,9 @@
 // Scoring, not counting, bounds searches of few samples: at 1000 SNPs x 4000
 // samples the matrix cores need 1.4 ms, and a search that derived both
 // classes' 27 integer cells of every triplet before it bounded its score took
-// 7.3 ms (540 vector instructions per triplet beside the contraction's, and
-// 57% of the wave time waiting for its table gathers).  Nearly every triplet
-// only has to be shown not to matter, so that is what the first pass does, in
-// FP32 from what the accumulators already hold:
+// 4.45 ms (540 vector instructions per triplet beside the contraction's).
+// Nearly every triplet only has to be shown not to matter, so that is what the
+// first pass does, in FP32 from what the accumulators already hold:
 //  * a lane keeps one Z, so its (X, Z) pair tables are registers of the whole
 //    unit, the (X, Y) ones broadcast LDS words made once per unit, and only
 //    the (Y, Z) ones are read per triplet, one triplet ahead;
@@ -16,10 +15,12 @@
 //    not for the two classes, since D^2 / T is all the bound needs;
 //  * 1 / T is one integer subtraction (recip_above).
 // That is about 250 instructions per triplet: a search at 1000 x 4000 (MI)
-// takes 3.67 ms instead of 4.45, 777 x 20001 (K2, no signal, 30% cases) 6.46
-// instead of 7.21, 2048 x 262144 809 instead of 811.  Lanes whose triplet it cannot rule
+// took 3.67 ms with it, 777 x 20001 (K2, no signal, 30% cases) 6.46 instead of
+// 7.21, 2048 x 262144 809 instead of 811.  Lanes whose triplet it cannot rule
 // out are collected in a bit mask, and a second, rolled loop takes the exact
-// integer tables and the FP32 score for those alone.
+// integer tables and the FP32 score for those alone; with the scores
+// branch-free (badness_f32_flat) and the search seeded (kernels_seed.hpp)
+// the first is at 3.23 ms, the second at 6.05.
 #pragma once
 #include "kernels_valu.hpp"
 
