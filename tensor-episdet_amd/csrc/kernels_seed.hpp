@@ -35,8 +35,22 @@ struct SeedArgs {
     float *s32;                         // top-k: badness of triplet (pair, c) at pair * n + c, else null
 };
 
-__global__ __launch_bounds__(256) void k_seed_pairs(SeedArgs a)
+// The 3-way jobs of a batch are seeded together, job by blockIdx.y, in grids
+// sized for the largest.  Without a bound, every workgroup that reaches a
+// job's first units scores all their triplets.  8 2-way and 8 3-way jobs
+// of 233 to 700 SNPs and 6667 to 20000 samples took 11.8 ms; with the seeds
+// (75 us for the 8 jobs), candidates staged by the re-scoring kernel and
+// group lists kept on the device 8.9 ms.
+struct SeedMany {
+    const SeedArgs *jobs;
+};
+__device__ __forceinline__ const SeedArgs &seed_args(const SeedArgs &a) { return a; }
+__device__ __forceinline__ SeedArgs seed_args(const SeedMany &m) { return ld_const(m.jobs, (size_t)blockIdx.y); }
+
+template <class Args>
+__global__ __launch_bounds__(256) void k_seed_pairs(Args args)
 {
+    const SeedArgs &a = seed_args(args);
     __shared__ unsigned long long s_k[4], s_p[4];
     const int n = a.r.n, tid = threadIdx.x;
     const float pi = a.sc.lb_pi;
@@ -68,7 +82,7 @@ __global__ __launch_bounds__(256) void k_seed_pairs(SeedArgs a)
         s_p[tid >> 6] = pk;
     }
     __syncthreads();
-    if (tid == 0) {
+    if (tid == 0 && (int)blockIdx.x < a.blocks) {
         for (int w = 1; w < 4; w++)
             if (lex_less(s_k[w], s_p[w], key, pk)) {
                 key = s_k[w];
@@ -79,8 +93,10 @@ __global__ __launch_bounds__(256) void k_seed_pairs(SeedArgs a)
     }
 }
 
-__global__ __launch_bounds__(SEED_BLOCKS) void k_seed_pick(SeedArgs a)
+template <class Args>
+__global__ __launch_bounds__(SEED_BLOCKS) void k_seed_pick(Args args)
 {
+    const SeedArgs &a = seed_args(args);
     __shared__ unsigned long long s_k[16], s_p[16];
     const int t = threadIdx.x, w = t >> 6;
     unsigned long long key = ~0ull, pk = ~0ull;
@@ -110,8 +126,10 @@ __global__ __launch_bounds__(SEED_BLOCKS) void k_seed_pick(SeedArgs a)
 }
 
 // One wave per (pair, c); c runs over all SNPs, so pair * n + c below npairs * n.
-__global__ __launch_bounds__(256) void k_seed_triplets(SeedArgs a)
+template <class Args>
+__global__ __launch_bounds__(256) void k_seed_triplets(Args args)
 {
+    const SeedArgs &a = seed_args(args);
     __shared__ float s_lnf[LNF_SMALL];
     __shared__ float s_min[4];
     load_lnf(s_lnf);

@@ -1136,16 +1136,23 @@ __global__ __launch_bounds__(64) void k_rescore_after(RescoreArgs p, const unsig
 }
 
 // FP64 re-scoring of the candidates of many searches; the candidate counts
-// are read on the device, so the whole batch needs no host round trip.
+// are read on the device and the outcomes go to the jobs' pinned staging areas,
+// so the whole batch needs no host round trip.
 struct RescoreJob {
     RescoreArgs r;                 // r.count unused
     const unsigned *count;         // candidates appended by the search, and the
                                    // overflow flag (CandOut::cand_count)
     unsigned cap;                  // buffer capacity (larger counts: overflow)
+    const float *cand_s32;
+    HostStage hs;                  // the job's pinned staging area, as in k_rescore_after
 };
 
 __global__ __launch_bounds__(64) void k_rescore_batch(const RescoreJob *jobs, int njobs)
 {
+    for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < njobs; k += (int)(gridDim.x * blockDim.x)) {
+        jobs[k].hs.ctl[0] = jobs[k].count[0];
+        jobs[k].hs.ctl[1] = jobs[k].count[1];
+    }
     for (unsigned long long gi = blockIdx.x;; gi += gridDim.x) {
         unsigned long long start = 0;
         int j = 0;
@@ -1156,7 +1163,13 @@ __global__ __launch_bounds__(64) void k_rescore_batch(const RescoreJob *jobs, in
             start += cnt;
         }
         if (j == njobs) return;
-        rescore_one(jobs[j].r, (int)(gi - start));
+        const unsigned i = (unsigned)(gi - start);
+        const double v = rescore_one(jobs[j].r, (int)i);
+        if (threadIdx.x == 0 && i < jobs[j].hs.slots) {
+            jobs[j].hs.packed[i] = jobs[j].r.cand[i];
+            jobs[j].hs.s32[i] = jobs[j].cand_s32[i];
+            jobs[j].hs.s64[i] = v;
+        }
     }
 }
 

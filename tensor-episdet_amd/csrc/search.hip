@@ -1006,6 +1006,25 @@ unsigned long long *stage_packed(unsigned char *base) { return (unsigned long lo
 float *stage_s32(unsigned char *base) { return (float *)(base + 256 + 8 * (size_t)STAGE_CAND); }
 double *stage_s64(unsigned char *base) { return (double *)(base + 256 + 12 * (size_t)STAGE_CAND); }
 
+HostStage host_stage(episdet_dataset *ds, unsigned cap)
+{
+    HostStage hs;
+    hs.ctl = stage_ctl(ds->stage_dev);
+    hs.packed = stage_packed(ds->stage_dev);
+    hs.s32 = stage_s32(ds->stage_dev);
+    hs.s64 = stage_s64(ds->stage_dev);
+    hs.slots = std::min<unsigned>(cap, STAGE_CAND);
+    return hs;
+}
+
+// Adds the `count` candidates a search left: from the staging area if they
+// all fit it.
+int collect_staged(episdet_dataset *ds, int count, Collected &acc)
+{
+    if (count > (int)STAGE_CAND) return collect(ds, count, acc);
+    return collect_host(stage_packed(ds->stage), stage_s32(ds->stage), stage_s64(ds->stage), count, acc);
+}
+
 // Writes the gathered winner (and, for top-k, the ranking) into res and ds.
 int finish(episdet_dataset *ds, int order, const Collected &acc, episdet_result *res)
 {
@@ -1028,12 +1047,12 @@ int finish(episdet_dataset *ds, int order, const Collected &acc, episdet_result 
     return EPISDET_OK;
 }
 
-// Winner of `count` candidates already re-scored on the device.
+// Winner of `count` candidates already re-scored and staged by the device.
 int collect_best(episdet_dataset *ds, int order, int score, int count, episdet_result *res)
 {
     Collected acc;
     acc.score = score;
-    CHK(collect(ds, count, acc));
+    CHK(collect_staged(ds, count, acc));
     return finish(ds, order, acc, res);
 }
 
@@ -1149,24 +1168,30 @@ unsigned long long unit_sets_max(const FusedPlan &pl)
 // become candidates; the score bounds then skip FP32 scores from the first unit on when
 // strongly associated triplets have associated pairs.
 constexpr int SEED_PAIRS = 4;
-int seed_from_pairs(episdet_dataset *ds, const FusedPlan &pl, int topk)
+SeedArgs seed_args_of(episdet_dataset *ds, int score, const ScoreCtx &sc, int npairs, bool topk)
 {
     SeedArgs a;
     std::memset(&a, 0, sizeof a);
-    a.r = rescore_args(ds, 3, pl.score);
+    a.r = rescore_args(ds, 3, score);
     a.r.cand = nullptr;
     a.r.out_s64 = nullptr;
-    a.sc = pl.sc;
+    a.sc = sc;
     a.blk = ds->seed;
     a.pick = ds->seed + 2 * SEED_BLOCKS;
     a.blocks = std::min(SEED_BLOCKS, ds->n - 1);
-    a.npairs = pl.seed_pairs;
+    a.npairs = npairs;
     a.best_key = &ds->ctl->best32;
     a.s32 = topk ? ds->cand_s32 : nullptr;     // free until the search appends
+    return a;
+}
+
+int seed_from_pairs(episdet_dataset *ds, const FusedPlan &pl, int topk)
+{
+    const SeedArgs a = seed_args_of(ds, pl.score, pl.sc, pl.seed_pairs, topk != 0);
     const int m = a.npairs * ds->n;
-    hipLaunchKernelGGL(k_seed_pairs, dim3(a.blocks), dim3(256), 0, ds->stream, a);
-    hipLaunchKernelGGL(k_seed_pick, dim3(1), dim3(SEED_BLOCKS), 0, ds->stream, a);
-    hipLaunchKernelGGL(k_seed_triplets, dim3((m + 3) / 4), dim3(256), 0, ds->stream, a);
+    hipLaunchKernelGGL(k_seed_pairs<SeedArgs>, dim3(a.blocks), dim3(256), 0, ds->stream, a);
+    hipLaunchKernelGGL(k_seed_pick<SeedArgs>, dim3(1), dim3(SEED_BLOCKS), 0, ds->stream, a);
+    hipLaunchKernelGGL(k_seed_triplets<SeedArgs>, dim3((m + 3) / 4), dim3(256), 0, ds->stream, a);
     if (topk)
         hipLaunchKernelGGL(k_seed_kth, dim3(1), dim3(1024), 0, ds->stream, ds->cand_s32, m, (unsigned)topk,
                            &ds->ctl->best32);
@@ -1264,12 +1289,7 @@ int launch_fused_rescored(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned
     int rc = issue_fused(ds, pl, topk, 0, pl.nunits, cap, seed_key, ds->ev[0], ds->ev[1]);
     if (rc == EPISDET_OK) {
         const RescoreArgs r = rescore_args(ds, pl.order, pl.score);
-        HostStage hs;
-        hs.ctl = stage_ctl(ds->stage_dev);
-        hs.packed = stage_packed(ds->stage_dev);
-        hs.s32 = stage_s32(ds->stage_dev);
-        hs.s64 = stage_s64(ds->stage_dev);
-        hs.slots = std::min<unsigned>(cap, STAGE_CAND);
+        const HostStage hs = host_stage(ds, cap);
         const unsigned grid = std::min<unsigned>(cap, 16u * (unsigned)ds->cu);
         hipLaunchKernelGGL(k_rescore_after, dim3(grid), dim3(64), 0, ds->stream, r, &ds->ctl->cand_count, cap,
                            (const float *)ds->cand_s32, hs);
@@ -1633,10 +1653,7 @@ int run_fused(episdet_dataset *ds, const episdet_options *o, episdet_result *res
         // re-scored on the device behind the search; the first STAGE_CAND
         // candidates are already on the host
         rms_total = rms;
-        const int count = (int)hc.cand_count;
-        if (count <= (int)STAGE_CAND)
-            CHK(collect_host(stage_packed(ds->stage), stage_s32(ds->stage), stage_s64(ds->stage), count, acc));
-        else CHK(collect(ds, count, acc));
+        CHK(collect_staged(ds, (int)hc.cand_count, acc));
     } else {
         // more sets within the FP32 margin than slots: search again in
         // windows, from the bound that the launch arrived at
@@ -2360,9 +2377,6 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         ktile[j] = o.tile;
         if (o.path == EPISDET_PATH_AUTO) CHK(choose_kernel(ds, o.order, o.score, &kpath[j], &ktile[j], o.autotune != 0));
     }
-    // the count tables are built on the datasets' streams, side by side; the
-    // graph runs on its own
-    for (int j = 0; j < njobs; j++) HIPCHK(hipStreamSynchronize(dss[j]->stream));
     // AUTO jobs of one order share one kernel: the MFMA tile their per-shape
     // choices give the most work (sets x samples).  One graph branch per order
     // packs the CUs better than one branch per tile: on the 64-job workload
@@ -2409,27 +2423,33 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
     // per-job kernel arguments
     std::vector<TriArgs> ta[MFMA_TILES];
     std::vector<unsigned long long> tstart[MFMA_TILES];
+    std::vector<SeedArgs> seeds;
+    int seed_blocks = 0, seed_sets = 0;
     for (int tl = 0; tl < MFMA_TILES; tl++) {
         ta[tl].resize(tri[tl].size());
         tstart[tl].assign(1, 0ull);
         for (size_t k = 0; k < tri[tl].size(); k++) {
             episdet_dataset *ds = dss[tri[tl][k]];
-            std::vector<int2> groups;
-            std::vector<unsigned long long> gstart;
-            build_groups(ds->n, mfma_ty(tl), mfma_tz(tl), groups, gstart, mfma_xstep(tl));
-            unsigned long long *d_gstart;
-            int2 *d_groups;
-            CHK(dl.put(&d_gstart, gstart.data(), gstart.size()));
-            CHK(dl.put(&d_groups, groups.data(), groups.size()));
+            const int t[3] = {mfma_ty(tl), mfma_tz(tl), mfma_xstep(tl)};
+            int ngroups;
+            unsigned long long nunits;
+            CHK(ensure_groups(ds, t, &ngroups, &nunits));
             TriArgs &a = ta[tl][k];
             fill_tri_common(ds, a);
             a.co.cand_cap = batch_cap(opts[tri[tl][k]], 3, tl);
             a.sc = make_ctx(ds, opts[tri[tl][k]].score, 3);
-            a.gstart = d_gstart;
-            a.groups = d_groups;
-            a.ngroups = (int)groups.size();
-            a.nunits = gstart.back();
-            tstart[tl].push_back(tstart[tl].back() + gstart.back());
+            a.gstart = ds->gstart;
+            a.groups = ds->groups;
+            a.ngroups = ngroups;
+            a.nunits = nunits;
+            tstart[tl].push_back(tstart[tl].back() + nunits);
+            const int np = seed_pairs(ds, 0, false);
+            if (np > 0) {
+                seeds.push_back(seed_args_of(ds, opts[tri[tl][k]].score, a.sc, np, false));
+                seed_blocks = std::max(seed_blocks, seeds.back().blocks);
+                seed_sets = std::max(seed_sets, np * ds->n);
+            }
+            results[tri[tl][k]].seeded = np > 0;
         }
     }
     std::vector<PairArgs> pa[MFMA_PAIR_TILES];
@@ -2453,24 +2473,11 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
     std::vector<unsigned *> bp(batched.size()), cp(batched.size());
     for (size_t k = 0; k < batched.size(); k++) {
         episdet_dataset *ds = dss[batched[k]];
-        RescoreArgs &r = rj[k].r;
-        std::memset(&r, 0, sizeof r);
-        r.p0 = ds->planes[0];
-        r.p1 = ds->planes[1];
-        r.W0 = ds->W[0];
-        r.W1 = ds->W[1];
-        r.n = ds->n;
-        r.N0 = ds->N[0];
-        r.N1 = ds->N[1];
-        r.order = opts[batched[k]].order;
-        r.score = opts[batched[k]].score;
-        r.singles = ds->singles;
-        r.pairs = ds->pairs;
-        r.t64 = ds->tab[r.score].t64;
-        r.cand = ds->cand;
-        r.out_s64 = ds->cand_s64;
+        rj[k].r = rescore_args(ds, opts[batched[k]].order, opts[batched[k]].score);
         rj[k].count = &ds->ctl->cand_count;
-        rj[k].cap = batch_cap(opts[batched[k]], r.order, ktile[batched[k]]);
+        rj[k].cap = batch_cap(opts[batched[k]], opts[batched[k]].order, ktile[batched[k]]);
+        rj[k].cand_s32 = ds->cand_s32;
+        rj[k].hs = host_stage(ds, rj[k].cap);
         qp[k] = ds->ctl->queue;
         bp[k] = &ds->ctl->best32;
         cp[k] = &ds->ctl->cand_count;
@@ -2479,33 +2486,45 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
     PairArgs *d_pa[MFMA_PAIR_TILES] = {};
     unsigned long long *d_tstart[MFMA_TILES] = {}, *d_pstart[MFMA_PAIR_TILES] = {}, *d_bq = nullptr;
     RescoreJob *d_rj = nullptr;
+    SeedArgs *d_seeds = nullptr;
     unsigned long long **d_qp = nullptr;
     unsigned **d_bp = nullptr, **d_cp = nullptr;
     constexpr int NQ = MFMA_TILES + MFMA_PAIR_TILES;   // one work queue per batched kernel
     constexpr int QW = 9 * QLINE;                      // each: the queue, then 8 per-XCD queues
     const std::vector<unsigned long long> zeros(NQ * QW, 0ull);
     for (int tl = 0; tl < MFMA_TILES; tl++) {
+        if (tri[tl].empty()) continue;
         CHK(dl.put(&d_ta[tl], ta[tl].data(), ta[tl].size()));
         CHK(dl.put(&d_tstart[tl], tstart[tl].data(), tstart[tl].size()));
     }
     for (int tl = 0; tl < MFMA_PAIR_TILES; tl++) {
+        if (pairs[tl].empty()) continue;
         CHK(dl.put(&d_pa[tl], pa[tl].data(), pa[tl].size()));
         CHK(dl.put(&d_pstart[tl], pstart[tl].data(), pstart[tl].size()));
     }
     CHK(dl.put(&d_bq, zeros.data(), zeros.size()));
+    CHK(dl.put(&d_seeds, seeds.data(), seeds.size()));
     CHK(dl.put(&d_rj, rj.data(), rj.size()));
     CHK(dl.put(&d_qp, qp.data(), qp.size()));
     CHK(dl.put(&d_bp, bp.data(), bp.size()));
     CHK(dl.put(&d_cp, cp.data(), cp.size()));
 
+    // the count tables and group lists are built on the datasets' streams,
+    // side by side; the graph runs on its own
+    for (int j = 0; j < njobs; j++) HIPCHK(hipStreamSynchronize(dss[j]->stream));
     double gms = 0;
     if (!batched.empty()) {
         hipStream_t st, br[NQ];
         HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        for (int q = 0; q < NQ; q++) HIPCHK(hipStreamCreateWithFlags(&br[q], hipStreamNonBlocking));
-        hipEvent_t fork, join[NQ];
+        const auto used = [&](int q) { return !(q < MFMA_TILES ? tri[q] : pairs[q - MFMA_TILES]).empty(); };
+        hipEvent_t fork, seeded, join[NQ];
         HIPCHK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
-        for (int q = 0; q < NQ; q++) HIPCHK(hipEventCreateWithFlags(&join[q], hipEventDisableTiming));
+        HIPCHK(hipEventCreateWithFlags(&seeded, hipEventDisableTiming));
+        for (int q = 0; q < NQ; q++)
+            if (used(q)) {
+                HIPCHK(hipStreamCreateWithFlags(&br[q], hipStreamNonBlocking));
+                HIPCHK(hipEventCreateWithFlags(&join[q], hipEventDisableTiming));
+            }
         hipGraph_t graph;
         hipGraphExec_t exec;
         // one graph: reset, then one branch per batched kernel (each 3-way
@@ -2516,9 +2535,24 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         hipLaunchKernelGGL(k_init_many, dim3((std::max(nb, NQ * QW) + 63) / 64), dim3(64), 0, st, d_qp, d_bp, d_cp, nb,
                            d_bq, NQ * QW);
         HIPCHK(hipEventRecord(fork, st));
-        for (int q = 0; q < NQ; q++) HIPCHK(hipStreamWaitEvent(br[q], fork, 0));
+        for (int q = 0; q < NQ; q++)
+            if (used(q)) HIPCHK(hipStreamWaitEvent(br[q], fork, 0));
+        // the 3-way jobs' starting bounds, beside the 2-way kernels, whose
+        // workgroups so get their CUs first: started together with the
+        // 3-way ones they held LDS for 9.2 ms to do 0.1 ms of work
+        if (!seeds.empty()) {
+            for (size_t k = 0; k < seeds.size(); k += 65535) {       // a grid's y extent
+                const SeedMany sm{d_seeds + k};
+                const unsigned nj = (unsigned)std::min<size_t>(seeds.size() - k, 65535);
+                hipLaunchKernelGGL(k_seed_pairs<SeedMany>, dim3(seed_blocks, nj), dim3(256), 0, st, sm);
+                hipLaunchKernelGGL(k_seed_pick<SeedMany>, dim3(1, nj), dim3(SEED_BLOCKS), 0, st, sm);
+                hipLaunchKernelGGL(k_seed_triplets<SeedMany>, dim3((seed_sets + 3) / 4, nj), dim3(256), 0, st, sm);
+            }
+            HIPCHK(hipEventRecord(seeded, st));
+        }
         for (int tl = 0; tl < MFMA_TILES; tl++) {
             if (tri[tl].empty()) continue;
+            if (!seeds.empty()) HIPCHK(hipStreamWaitEvent(br[tl], seeded, 0));
             BatchTri bt;
             bt.jobs = d_ta[tl];
             bt.job_start = d_tstart[tl];
@@ -2543,6 +2577,7 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
                 br[MFMA_TILES + tl]);
         }
         for (int q = 0; q < NQ; q++) {
+            if (!used(q)) continue;
             HIPCHK(hipEventRecord(join[q], br[q]));
             HIPCHK(hipStreamWaitEvent(st, join[q], 0));
         }
@@ -2555,7 +2590,7 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         HIPCHK(hipEventRecord(e0, st));
         HIPCHK(hipGraphLaunch(exec, st));
         HIPCHK(hipEventRecord(e1, st));
-        HIPCHK(hipEventSynchronize(e1));
+        HIPCHK(hipStreamSynchronize(st));
         float f = 0;
         HIPCHK(hipEventElapsedTime(&f, e0, e1));
         gms = f;
@@ -2564,7 +2599,9 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
         (void)hipGraphExecDestroy(exec);
         (void)hipGraphDestroy(graph);
         (void)hipEventDestroy(fork);
+        (void)hipEventDestroy(seeded);
         for (int q = 0; q < NQ; q++) {
+            if (!used(q)) continue;
             (void)hipEventDestroy(join[q]);
             (void)hipStreamDestroy(br[q]);
         }
@@ -2573,14 +2610,13 @@ int episdet_run_batch(episdet_dataset *const *dss, const episdet_options *opts, 
     for (size_t k = 0; k < batched.size(); k++) {
         const int j = batched[k];
         episdet_dataset *ds = dss[j];
-        Ctl hc;
-        HIPCHK(hipMemcpy(&hc, ds->ctl, sizeof hc, hipMemcpyDeviceToHost));
-        if (hc.cand_count == 0 || hc.cand_over || hc.cand_count > batch_cap(opts[j], opts[j].order, ktile[j])) {
+        const unsigned count = stage_ctl(ds->stage)[0], over = stage_ctl(ds->stage)[1];
+        if (count == 0 || over || count > batch_cap(opts[j], opts[j].order, ktile[j])) {
             solo.push_back(j);     // overflow: exact rerun on its own
             continue;
         }
         episdet_result &r = results[j];
-        CHK(collect_best(ds, opts[j].order, opts[j].score, (int)hc.cand_count, &r));
+        CHK(collect_best(ds, opts[j].order, opts[j].score, (int)count, &r));
         // the graph's device time; its re-scoring kernel is part of it
         // (rescore_ms stays 0 for batched jobs)
         r.kernel_ms = gms;

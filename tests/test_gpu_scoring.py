@@ -48,6 +48,31 @@ def test_pair_unit_edges(n, Nc, Nt, score):
             assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
 
 
+@pytest.mark.parametrize("score", [episdet.K2, episdet.MI])
+def test_batch_seeds_every_three_way_job(score):
+    """The 3-way jobs of a batch are seeded in grids sized for the largest one:
+    one triplet (not seeded), the smallest seeded job, larger ones with 2-way jobs
+    between, and more SNPs than the pair ranking has workgroups (1024)."""
+    sizes = [(3, 3, 40), (2, 90, 700), (3, 4, 1030), (3, 65, 900), (2, 5, 64), (3, 130, 300)]
+    syns = [episdet.generate(n, N // 3, N - N // 3, seed=500 + j, planted_sets=int(n >= 64), planted_order=o)
+            for j, (o, n, N) in enumerate(sizes)]
+    ref = [O.search(s.cases, s.controls, s.num_cases, s.num_controls, o, score) for (o, _, _), s in zip(sizes, syns)]
+    # too many triplets for the oracle: the search without a starting bound is the reference
+    sizes.append((3, 1030, 200))
+    syns.append(episdet.generate(1030, 90, 110, seed=550))
+    dss = [episdet.Dataset.from_synthetic(s) for s in syns]
+    r = dss[-1].run_noalloc(3, score)
+    ref.append({"packed": r["packed"], "score": r["best_score"]})
+    for rep in range(3):
+        print(f"batch score={score} rep={rep}", flush=True)
+        res, _ = episdet.run_batch(dss, [o for o, _, _ in sizes], [score] * len(sizes), rebuild=rep == 1)
+        assert [x["seeded"] for x in res] == [int(o == 3 and n > 3) for o, n, _ in sizes]
+        for x, o in zip(res, ref):
+            assert x["packed"] == o["packed"] and x["best_score"] == o["score"]
+    for d in dss:
+        d.close()
+
+
 def test_upload_through_the_pinned_pool():
     """Planes of 4 MB and more a class go to the device in chunks of whole SNPs
     (239 of them here); the rows on both sides of a chunk's edge, the caller's
