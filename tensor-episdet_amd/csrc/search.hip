@@ -702,9 +702,14 @@ int launch_pairs_batch(int R, int cu, const BatchPair &bp, hipStream_t s)
     if (R == 4) {
         int grid = launch_blocks((const void *)k_pairs_valu<4, MODE>, cu);
         hipLaunchKernelGGL((k_pairs_valu<4, MODE>), dim3(grid), dim3(256), 0, s, bp);
-    } else {
+    } else if (R == 2) {
         int grid = launch_blocks((const void *)k_pairs_valu<2, MODE>, cu);
         hipLaunchKernelGGL((k_pairs_valu<2, MODE>), dim3(grid), dim3(256), 0, s, bp);
+    } else if constexpr (MODE == MODE_SEARCH) {
+        int grid = launch_blocks((const void *)k_pairs_valu<1, MODE>, cu);
+        hipLaunchKernelGGL((k_pairs_valu<1, MODE>), dim3(grid), dim3(256), 0, s, bp);
+    } else {
+        return EPISDET_ERR_INTERNAL;
     }
     HIPCHK(hipGetLastError());
     return EPISDET_OK;
@@ -743,7 +748,7 @@ int launch_pairs_mfma(int tile, int blocks, const BatchPair &bp, hipStream_t s)
 void fill_pairs(episdet_dataset *ds, PairArgs &a, bool mfma, int tile);
 
 template <int MODE>
-int dispatch_pairs(episdet_dataset *ds, bool mfma, int tile, PairArgs &a, hipStream_t s)
+int dispatch_pairs(episdet_dataset *ds, bool mfma, int tile, PairArgs &a, hipStream_t s, int R = 0)
 {
     BatchPair bp;
     bp.jobs = (const PairArgs *)ds->jobargs;
@@ -760,7 +765,7 @@ int dispatch_pairs(episdet_dataset *ds, bool mfma, int tile, PairArgs &a, hipStr
             per = 1;
         return launch_pairs_mfma<MODE>(tile, per * ds->cu, bp, s);
     }
-    return launch_pairs_batch<MODE>(PAIR_TILES[tile], ds->cu, bp, s);
+    return launch_pairs_batch<MODE>(R ? R : PAIR_TILES[tile], ds->cu, bp, s);
 }
 
 // Groups of 3-way units: (Y tile, Z tile) pairs that hold at least one
@@ -1066,6 +1071,7 @@ struct FusedPlan {
     ScoreCtx sc{};
     unsigned long long nunits = 0;
     unsigned seed_key = 0;       // starting global bound (best32), 0: none
+    int pr = 0;                  // VALU 2-way: units of 16 pr x 16 pr
     int seed_pairs = 0;          // 3-way: > 0: the launch starts from the triplets of this many best pairs
     void group_tile(int (&t)[3]) const
     {
@@ -1119,7 +1125,7 @@ bool tile_valid(int order, int path, int tile)
 }
 
 // Tables, pair table and candidate buffer must exist (ensure_*) before.
-int plan_fused(episdet_dataset *ds, int order, int score, int path, int tile, FusedPlan &pl)
+int plan_fused(episdet_dataset *ds, int order, int score, int path, int tile, FusedPlan &pl, int topk = 0)
 {
     pl.order = order;
     pl.score = score;
@@ -1141,6 +1147,21 @@ int plan_fused(episdet_dataset *ds, int order, int score, int path, int tile, Fu
         pl.ta.nunits = pl.nunits;
     } else {
         fill_pairs(ds, pl.pa, pl.mfma, tile);
+        if (!pl.mfma) {
+            pl.pr = PAIR_TILES[tile];
+            // VALU tile 1 with at most 3/2 units of 16 x 16 a CU (432 SNPs):
+            // units of that size, one pair a thread, so a quarter of the serial
+            // work each.  A search, 32 x 32 and 16 x 16 units: 53 and 49 us at
+            // 64 x 500, 63 and 57 at 400 x 4000, 61 and 53 at 256 x 4096 (MI).
+            // From two units a CU their turns cost more: 57 and 60 us at 512 x
+            // 2048, 59 and 65 at 640 x 2000.  Not for top-k, which may ask for
+            // 1024 sets of a unit.
+            const unsigned long long t = (unsigned long long)(ds->n + 15) / 16, u = t * (t + 1) / 2;
+            if (pl.pr == 2 && !topk && 2 * u <= 3ull * (unsigned long long)ds->cu) {
+                pl.pr = 1;
+                fill_pair_common(ds, pl.pa, 16);
+            }
+        }
         pl.pa.sc = pl.sc;
         pl.nunits = pl.pa.nunits;
     }
@@ -1257,7 +1278,7 @@ int issue_fused(episdet_dataset *ds, FusedPlan &pl, int topk, unsigned long long
     else
         rc = order == 3 ? (mfma ? dispatch_tri_mfma<MODE_SEARCH>(ds, tile, ta, ds->stream)
                                 : dispatch_tri<MODE_SEARCH>(ds, tile, ta, 0, ds->stream))
-                        : dispatch_pairs<MODE_SEARCH>(ds, mfma, tile, pa, ds->stream);
+                        : dispatch_pairs<MODE_SEARCH>(ds, mfma, tile, pa, ds->stream, pl.pr);
     HIPCHK(hipEventRecord(e1, ds->stream));
     return rc;
 }
@@ -1390,8 +1411,8 @@ unsigned long long count_sets(const episdet_dataset *ds, const FusedPlan &pl, un
         }
     } else {
         const bool p2 = pl.mfma && pl.tile == 0;   // 128 x 64 order; the others are triangular
-        const long long TA = p2 ? P2_TA : (pl.mfma ? P3_TA : 16 * PAIR_TILES[pl.tile]);
-        const long long TB = p2 ? P2_TB : (pl.mfma ? P3_TB : 16 * PAIR_TILES[pl.tile]);
+        const long long TA = p2 ? P2_TA : (pl.mfma ? P3_TA : 16 * pl.pr);
+        const long long TB = p2 ? P2_TB : (pl.mfma ? P3_TB : 16 * pl.pr);
         for (unsigned long long u = u0; u < u1; u++) {
             long long ta, tb;
             if (p2 && pl.pa.blocked) {
@@ -1441,7 +1462,8 @@ unsigned long long resident_blocks(const episdet_dataset *ds, const FusedPlan &p
     if (pl.mfma)
         return (unsigned long long)occupancy_blocks(pairs_mfma_kernel<MODE_SEARCH>(pl.tile), pairs_mfma_threads(pl.tile),
                                                     cu);
-    if (PAIR_TILES[pl.tile] == 2) return (unsigned long long)launch_blocks((const void *)k_pairs_valu<2, MODE_SEARCH>, cu);
+    if (pl.pr == 1) return (unsigned long long)launch_blocks((const void *)k_pairs_valu<1, MODE_SEARCH>, cu);
+    if (pl.pr == 2) return (unsigned long long)launch_blocks((const void *)k_pairs_valu<2, MODE_SEARCH>, cu);
     return (unsigned long long)launch_blocks((const void *)k_pairs_valu<4, MODE_SEARCH>, cu);
 }
 
@@ -1626,7 +1648,7 @@ int run_fused(episdet_dataset *ds, const episdet_options *o, episdet_result *res
     if (order == 3) CHK(ensure_pairs(ds));
     if (path == EPISDET_PATH_AUTO) CHK(choose_kernel(ds, order, score, &path, &tile, o->autotune != 0, true));
     FusedPlan pl;
-    CHK(plan_fused(ds, order, score, path, tile, pl));
+    CHK(plan_fused(ds, order, score, path, tile, pl, topk));
     // Candidate slots of this search: the requested capacity, by default 1M
     // and for top-k at least what the resident blocks append before the
     // bound settles (about 2k sets each); never fewer than one work unit's

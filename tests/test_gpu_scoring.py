@@ -73,6 +73,24 @@ def test_batch_seeds_every_three_way_job(score):
         d.close()
 
 
+@pytest.mark.parametrize("n,Nc,Nt", [(2, 1, 1), (16, 40, 25), (17, 1024, 1025), (432, 700, 300), (433, 300, 700)])
+@pytest.mark.parametrize("score", [episdet.K2, episdet.MI])
+def test_small_valu_pair_units(n, Nc, Nt, score):
+    """VALU pair tile 1 takes 16 x 16 units up to 432 SNPs (256 CUs) and 32 x 32
+    units beyond and for top-k; candidate_cap 64 forces windows of units."""
+    syn = episdet.generate(n, Nc, Nt, seed=600 + n, planted_sets=int(n >= 64), planted_order=2)
+    ref_p, ref_s = O.ranked(syn.cases, syn.controls, Nc, Nt, 2, score)
+    V = episdet.PATH_FUSED_VALU
+    with episdet.Dataset.from_synthetic(syn) as ds:
+        print(f"valu pair units n={n} Nc={Nc} Nt={Nt} score={score}", flush=True)
+        for r in (ds.run(2, score, path=V, tile=1), ds.run(2, score, path=V, tile=1, candidate_cap=64),
+                  ds.run_noalloc(2, score, path=V, tile=1)):
+            assert r["packed"] == int(ref_p[0]) and r["best_score"] == float(ref_s[0]) and r["tile"] == 1
+        m = min(1024, math.comb(n, 2))
+        p, s, _ = ds.topk(2, 1024, score=score, path=V, tile=1)
+        assert p == [int(x) for x in ref_p[:m]] and s == [float(x) for x in ref_s[:m]]
+
+
 def test_upload_through_the_pinned_pool():
     """Planes of 4 MB and more a class go to the device in chunks of whole SNPs
     (239 of them here); the rows on both sides of a chunk's edge, the caller's
